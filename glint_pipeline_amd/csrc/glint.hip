@@ -52,7 +52,19 @@ constexpr int kFineTile = 12288;                    // contacts per LDS tile of 
 constexpr uint32_t kMaxCoarse = 1024;               // coarse bins of pass 1
 constexpr uint32_t kMaxFine = 2048;                 // fine bins of pass 2
 constexpr int kBorderStage = 128;                   // staged border objects per wave (assign)
+// Counts of the join, kept in kJoinParts lines until k_bucket_count adds them up.
+enum JoinSum : uint32_t { kSumContacts, kSumBorder, kSumDup, kSumStored, kSumBand, kSumTests, kSumEvals, kJoinSums };
+constexpr uint32_t kJoinParts = 64;
+constexpr uint32_t kJoinPartStride = 16;            // 128 B
 constexpr uint32_t kHeavyLeaf = 256;                // leaves above this size are joined first
+constexpr uint32_t kSparseMax = 512;                // most objects of a leaf joined by one wave
+// and most objects per reach x reach square of it.  Denser leaves have
+// several contacts per object, which a wave decides one gather at a time and
+// the tiles in LDS: at 10M objects in hotspots a pass of 8 ticks takes 58.6 ms
+// at 0.06 and 0.25, 61 at 1 and 66 at 4; 400k objects (8 ticks and a flush)
+// 8.6, 8.5, 8.6 and 9.2 ms; 3000 objects at 0.012 a square metre 0.42, 0.40,
+// 0.40 and 0.39 ms.
+constexpr double kSparseDensity = 0.25;
 
 // ------------------------------------------------------------ predicates
 
@@ -416,6 +428,8 @@ __global__ void kf_stamp(const Many m)
 template <class P>
 __device__ __forceinline__ void reset_tick_body(const DevState s, const P blk)
 {
+    for (uint32_t k = threadIdx.x; k < kJoinParts * kJoinPartStride; k += blockDim.x) s.jpart[k] = 0;
+    if (threadIdx.x != 0) return;
     Counters *c = s.ctr;
     c->n_units = 0;
     c->n_contacts = 0;
@@ -431,6 +445,7 @@ __device__ __forceinline__ void reset_tick_body(const DevState s, const P blk)
     c->n_border = 0;
     c->n_leaf_list = 0;
     c->n_heavy = 0;
+    c->n_sparse = 0;
     c->n_leaves = 0;
     c->max_leaf = 0;
     c->n_drop_leaves = 0;
@@ -1502,10 +1517,26 @@ __global__ __launch_bounds__(kBlock) void kf_scan_objects(const Many m)
     scan_objects_body(m.ss[w.i], w.blk);
 }
 
+// The join's reach in the coordinates of a leaf's box, never less than the
+// distance the pair test accepts: planar, the reach with the guard band
+// around it; with geography, degrees of latitude, and degrees of longitude
+// at the leaf's latitude farthest from the equator (a pair's own point may
+// lie a reach outside the box).  The single-precision cosine is good to
+// 1e-5 below 89 degrees; higher leaves (x = 0) are left to the tiles.
+__device__ __forceinline__ double2 sparse_reach(const DevState &s, double ly, double hy)
+{
+    if (!s.geography) return make_double2(s.r + s.guard_reach, s.r + s.guard_reach);
+    const double ry = s.r * kDegPerMeterLat * (1.0 + 1e-9);
+    const double lat = fmax(fabs(ly), fabs(hy)) + ry;
+    if (lat > 89.0) return make_double2(0.0, ry);
+    return make_double2(s.r * (kDegPerMeterLat / (double)cosf((float)(lat * (kRefPi / 180.0)))) * (1.0 + 1e-4), ry);
+}
+
 // Unit offsets of every leaf, and the join work list: leaves with >= 2
 // objects (inside pairs) or with border units aimed at them.  Leaves of more
 // than kHeavyLeaf objects are listed from the back, so that the join takes
-// them first and ends on small leaves.
+// them first and ends on small leaves.  Sparse leaves, which the join gives
+// to one wave each (join_sparse), have a list of their own.
 template <class P>
 __device__ __forceinline__ void scan_units_body(const DevState s, const P blk)
 {
@@ -1524,11 +1555,21 @@ __device__ __forceinline__ void scan_units_body(const DevState s, const P blk)
         if (in) s.ustart[n] = ex;
         ex += c[k];
         const uint32_t cnt = in ? s.count[n] : 0u;
-        const bool work = in && (c[k] > 0 || cnt >= 2);
-        const bool heavy = work && cnt > kHeavyLeaf;
-        const uint32_t idx = wave_append_u32(&s.ctr->n_leaf_list, work && !heavy);
+        const bool work = in && cnt > 0 && (c[k] > 0 || cnt >= 2);
+        bool sparse = false;
+        if (work && cnt <= kSparseMax) {
+            const double2 lo = reinterpret_cast<const double2 *>(s.nodes + n)[1], hi = node_high(s.nodes, n);
+            const double2 r = sparse_reach(s, lo.y, hi.y);
+            sparse = (double)cnt * r.x * r.y <= kSparseDensity * (hi.x - lo.x) * (hi.y - lo.y) && r.x > 0.0;
+        }
+        const bool heavy = work && !sparse && cnt > kHeavyLeaf;
+        const uint32_t idx = wave_append_u32(&s.ctr->n_leaf_list, work && !heavy && !sparse);
         const uint32_t hdx = wave_append_u32(&s.ctr->n_heavy, heavy);
-        if (work) s.leaf_list[heavy ? s.node_cap - 1 - hdx : idx] = n;
+        const uint32_t sdx = wave_append_u32(&s.ctr->n_sparse, sparse);
+        if (sparse)
+            s.sparse_list[sdx] = n;
+        else if (work)
+            s.leaf_list[heavy ? s.node_cap - 1 - hdx : idx] = n;
     }
 }
 
@@ -1852,9 +1893,8 @@ struct TableShape {
     uint32_t bits, lo_bits, coarse;
 };
 
-__device__ __forceinline__ TableShape table_shape(const DevState &s)
+__device__ __forceinline__ TableShape table_shape(const DevState &s, unsigned long long n)
 {
-    const unsigned long long n = s.ctr->n_stored;
     uint32_t b = s.rbits_min;
     while (b < s.rbits_max && ((unsigned long long)kRegionFill << b) < n) b++;
     TableShape t;
@@ -1863,6 +1903,7 @@ __device__ __forceinline__ TableShape table_shape(const DevState &s)
     t.coarse = 1u << (b - t.lo_bits);
     return t;
 }
+__device__ __forceinline__ TableShape table_shape(const DevState &s) { return table_shape(s, s.ctr->n_stored); }
 
 // Contacts found by one wave are staged in LDS as (row lane, column) index
 // pairs and appended to the tick's contact list in 4096-entry chunks
@@ -2506,6 +2547,278 @@ struct JoinLds {
 };
 
 
+// ------------------------------------------------------- refine: sparse leaves
+//
+// A leaf whose objects are far apart (kSparseDensity) holds few pairs within
+// reach, and a 64 x 64 task over it tests pairs that are mostly far apart.
+// Such a leaf is joined by one wave: its objects are sorted into up to 16 x 16
+// cells no smaller than the reach (a counting sort in LDS), row by row, so
+// that the objects within reach of one lie in the rows of cells below, at and
+// above its own, in one run of the sorted order each.  An inside row tests
+// the rest of its run and the run above (each pair once); a border unit tests
+// all three.  The test in LDS is a single-precision one on offsets in units
+// of the reach, widened by its error so that it passes every contact; the
+// pairs that pass are staged, over all leaves of the wave, and the exact FP64
+// test, the key and its flags follow 64 pairs at a time, from the sorted
+// arrays: an object's ids and candidate lists are only read where a contact
+// needs them (the tiles read them for every object).
+// A leaf of 100 objects takes a wave about 5 us, nearly all of it waiting:
+// the leaf's record and positions (2 us), the sort (1.3), the runs (1.7).
+// The join of 1M uniform objects went from 297 to 39 us, of 300k in lon/lat
+// from 171 to 27, of 25.6M in 32 cities from 4.71 to 0.67 ms, of 20M served
+// from 3.2 to 0.5 ms.
+constexpr uint32_t kSparseSide = 16;
+constexpr uint32_t kSparseCells = kSparseSide * kSparseSide;
+constexpr uint32_t kSparseStage = 128;   // staged pairs, and stored keys, of a wave
+constexpr int kSparsePer = (int)(kSparseMax / 64);
+
+// A workgroup's counts, in the order of JoinSum.
+struct JoinSums {
+    unsigned long long of[kJoinSums];
+    unsigned long long base;         // its last keys' place in the contact list
+    uint32_t left[kBlock / 64];      // and their number per wave
+};
+
+struct SparseLds {
+    float2 pos[kSparseMax];               // offsets from the leaf's low corner in reaches, cell order
+    uint16_t at[kSparseMax];              // their place in the leaf's run of the sorted arrays
+    uint32_t start[kSparseCells + 4];     // first object of every cell, and the count at the end
+    uint2 stage[kSparseStage];            // staged pairs: row (sorted index, or unit), column (kSparseUnit: a unit row)
+    unsigned long long out[kSparseStage]; // keys of contacts to be stored
+};
+constexpr uint32_t kSparseUnit = 0x80000000u;
+
+// A wave's sums over its sparse leaves (per lane unless stated).
+struct SparseWave {
+    uint32_t n, nout;                  // staged pairs and keys (uniform)
+    uint32_t kept;                     // keys in all (uniform)
+    uint32_t pass_in, pass_bd;         // contacts
+    uint32_t band, dups;               // pairs in the guard band; found twice and not stored
+    unsigned long long tests, evals;   // evals: columns (uniform)
+};
+
+// Key of a staged pair, or kEmptyKey for one that is not a contact or not
+// stored: the decisions of join_columns' write-out, all of them in FP64.
+template <bool GEO>
+__device__ __forceinline__ unsigned long long sparse_key(const DevState &s, const TickView &tv, bool has_prev,
+                                                         SparseWave &w, uint2 e)
+{
+    const bool border = (e.y & kSparseUnit) != 0;
+    const uint32_t gj = e.y & ~kSparseUnit;
+    const uint4 ulf = border ? s.unit_lf[e.x] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t gi = border ? ulf.w : e.x;
+    const uint32_t pa = s.spid[gi], pb = s.spid[gj];
+    const double xi = tv.sx[gi], yi = tv.sy[gi], xj = tv.sx[gj], yj = tv.sy[gj];
+    double ex = xi - xj, ey = yi - yj;
+    if constexpr (GEO) {
+        ey = ey / kDegPerMeterLat;
+        ex = ex / s.sgeo[border || pa < pb ? gi : gj];
+    } else if (s.precision == GLINT_PRECISION_FP32_GUARD) {
+        // a pair that the FP32 test of the leaf's offsets does not decide counts as re-tested
+        const uint32_t leaf = s.tp->sleaf[gj];
+        const double2 lo = reinterpret_cast<const double2 *>(s.nodes + leaf)[1], hi = node_high(s.nodes, leaf);
+        const float s32 = dist2_f32((float)(xi - lo.x) - (float)(xj - lo.x), (float)(yi - lo.y) - (float)(yj - lo.y));
+        w.band += s32 > s.t32_in && s32 <= s.t32_out && hi.x - lo.x <= s.w32_max && hi.y - lo.y <= s.w32_max;
+    }
+    if (!(ex * ex + ey * ey <= s.t64)) return kEmptyKey;
+    w.pass_in += border ? 0u : 1u;
+    w.pass_bd += border ? 1u : 0u;
+    unsigned long long k = pair_key(pa, pb) | (border ? kTagBorder : 0ull);
+    if (has_prev) {
+        if (GEO) {
+            k |= kTagPrev;   // every contact is kept and looked up
+        } else {
+            const double dx = tv.xy_prev[2 * (size_t)pa] - tv.xy_prev[2 * (size_t)pb];
+            const double dy = tv.xy_prev[2 * (size_t)pa + 1] - tv.xy_prev[2 * (size_t)pb + 1];
+            if (dx * dx + dy * dy <= s.t64) k |= kTagPrev;
+        }
+    }
+    if (s.store_all) return k;
+    if (k & kTagPrev) {
+        // tested by the join of the tick before
+        const uint32_t la = border ? ulf.y : s.splf[gi], lb = s.splf[gj];
+        const uint4 ca = cand_at(s.tp->cand_prev, border ? ulf.z : s.sprev[gi], s.n, s.tp->prev_tick);
+        const uint4 cb = cand_at(s.tp->cand_prev, s.sprev[gj], s.n, s.tp->prev_tick);
+        const bool tested = (la == lb && la != kNone) ||
+                            (ca.w <= 3 && cb.w <= 3 &&
+                             (ca.x == lb || ca.y == lb || ca.z == lb || cb.x == la || cb.y == la || cb.z == la));
+        return tested ? k | kTagTested : k;
+    }
+    if (!border) return kEmptyKey;
+    const uint4 qc = cand_read(s.tp->cand, gj, s.tp->tick);
+    if ((ulf.x >> 31) || qc.w > 3) return k;
+    const uint32_t lp = ulf.x & 0x7FFFFFFFu;
+    w.dups += (qc.x == lp || qc.y == lp || qc.z == lp) && lp < s.tp->sleaf[gj];
+    return kEmptyKey;
+}
+
+// Stored keys [0, n) of a wave's buffer into the contact list at `base`.
+__device__ __forceinline__ void sparse_write(const DevState &s, const unsigned long long *out, uint32_t n,
+                                             unsigned long long base)
+{
+    unsigned long long *list = contact_out(s);
+    if (base + n > s.clist_cap) {
+        if (lane_id() == 0) atomicOr(&s.ctr->error, kErrContactCap);
+        return;
+    }
+    for (uint32_t i = lane_id(); i < n; i += 64) list[base + i] = out[i];
+}
+
+// Decides the last staged pairs (at most 64) and keeps the keys to be stored.
+template <bool GEO>
+__device__ __forceinline__ void sparse_drain(const DevState &s, const TickView &tv, bool has_prev, SparseLds &L,
+                                             SparseWave &w)
+{
+    wave_sync();
+    const uint32_t lane = lane_id(), m = min(w.n, 64u);
+    w.n -= m;
+    const unsigned long long key =
+        lane < m ? sparse_key<GEO>(s, tv, has_prev, w, L.stage[w.n + lane]) : kEmptyKey;
+    const unsigned long long keep = __builtin_amdgcn_ballot_w64(key != kEmptyKey);
+    if (key != kEmptyKey) L.out[w.nout + __popcll(keep & ((1ull << lane) - 1ull))] = key;
+    const uint32_t cnt = (uint32_t)__popcll(keep);
+    w.nout += cnt;
+    w.kept += cnt;
+    wave_sync();
+    if (w.nout > kSparseStage - 64) {
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&s.ctr->n_clist, (unsigned long long)w.nout);
+        sparse_write(s, L.out, w.nout, __shfl(base, 0));
+        wave_sync();
+        w.nout = 0;
+    }
+}
+
+template <bool GEO>
+__device__ __forceinline__ void join_sparse(const DevState &s, const TickView &tv, bool has_prev, SparseLds &L,
+                                            SparseWave &w, uint32_t leaf)
+{
+    const uint32_t lane = lane_id();
+    const uint32_t off = s.offset[leaf], cnt = s.count[leaf];
+    const uint32_t uoff = s.ustart[leaf], ucnt = s.ucount[leaf];
+    const double2 lo = reinterpret_cast<const double2 *>(s.nodes + leaf)[1], hi = node_high(s.nodes, leaf);
+    double x[kSparsePer], y[kSparsePer];
+#pragma unroll
+    for (int q = 0; q < kSparsePer; q++) {
+        const uint32_t k = lane + 64 * q;
+        x[q] = k < cnt ? tv.sx[off + k] : 0.0;
+        y[q] = k < cnt ? tv.sy[off + k] : 0.0;
+    }
+    // the first units' sorted positions, in flight meanwhile
+    uint32_t ug = lane < ucnt ? reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + lane)[3] : 0u;
+    wave_sync();
+    reinterpret_cast<uint4 *>(L.start)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    const double2 r = sparse_reach(s, lo.y, hi.y);
+    const double ix = 1.0 / r.x, iy = 1.0 / r.y;
+    const float nx = (float)((hi.x - lo.x) * ix), ny = (float)((hi.y - lo.y) * iy);
+    // An offset in reaches is rounded once (and its product in FP64), a
+    // difference, its square and their sum once more: below 2^-22 of the
+    // leaf's side (or a unit's offset, at most a reach outside it).
+    const float margin = 1e-6f * (fmaxf(nx, ny) + 4.0f);
+    const float lim = (1.0f + margin) * (1.0f + margin) * 1.000001f;
+    // cells at least a widened reach wide, so that objects within it differ
+    // by at most one cell each way (the cell number is monotone in the offset)
+    const float wide = 1.001f * (1.0f + margin);
+    const float gx = fminf(fmaxf(floorf(nx / wide), 1.0f), (float)kSparseSide);
+    const float gy = fminf(fmaxf(floorf(ny / wide), 1.0f), (float)kSparseSide);
+    const float kx = gx / nx, ky = gy / ny;
+    auto cell_of = [&](float2 p) {
+        return make_uint2((uint32_t)fminf(fmaxf(p.x * kx, 0.0f), gx - 1.0f),
+                          (uint32_t)fminf(fmaxf(p.y * ky, 0.0f), gy - 1.0f));
+    };
+    wave_sync();
+    float2 p[kSparsePer];
+    uint32_t at[kSparsePer];   // rank << 16 | cell
+#pragma unroll
+    for (int q = 0; q < kSparsePer; q++) {
+        p[q] = make_float2((float)((x[q] - lo.x) * ix), (float)((y[q] - lo.y) * iy));
+        at[q] = 0;
+        if (lane + 64 * q < cnt) {
+            const uint2 c = cell_of(p[q]);
+            const uint32_t cell = c.y * kSparseSide + c.x;
+            at[q] = atomicAdd(&L.start[cell], 1u) << 16 | cell;
+        }
+    }
+    wave_sync();
+    {
+        const uint4 c = reinterpret_cast<uint4 *>(L.start)[lane];
+        const uint32_t v = c.x + c.y + c.z + c.w;
+        const uint32_t before = wave_inclusive_scan(v) - v;
+        reinterpret_cast<uint4 *>(L.start)[lane] =
+            make_uint4(before, before + c.x, before + c.x + c.y, before + c.x + c.y + c.z);
+        if (lane == 0) L.start[kSparseCells] = cnt;
+    }
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < kSparsePer; q++) {
+        if (lane + 64 * q < cnt) {
+            const uint32_t d = L.start[at[q] & 0xFFFFu] + (at[q] >> 16);
+            L.pos[d] = p[q];
+            L.at[d] = (uint16_t)(lane + 64 * q);
+        }
+    }
+    wave_sync();
+    // The columns of a lane's row: up to three runs of the sorted order, one
+    // object per step and lane.
+    auto scan = [&](float2 row, uint32_t ex, uint32_t flag, uint32_t a0, uint32_t na, uint32_t b0, uint32_t nb,
+                    uint32_t c0, uint32_t nc) {
+        const uint32_t n = na + nb + nc;
+        const int dab = (int)b0 - (int)na, dbc = (int)c0 - (int)(na + nb);
+        for (uint32_t t = 0; __builtin_amdgcn_ballot_w64(t < n) != 0ull; t++) {
+            const bool live = t < n;
+            const uint32_t j = live ? (uint32_t)((int)t + (t < na ? (int)a0 : t < na + nb ? dab : dbc)) : 0u;
+            const float2 c = L.pos[j];
+            const float dx = row.x - c.x, dy = row.y - c.y;
+            const bool hit = live && dist2_f32(dx, dy) <= lim;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+            w.evals++;
+            if (!m) continue;
+            if (hit) L.stage[w.n + __popcll(m & ((1ull << lane) - 1ull))] = make_uint2(ex, (off + L.at[j]) | flag);
+            w.n += (uint32_t)__popcll(m);
+            if (w.n > kSparseStage - 64) sparse_drain<GEO>(s, tv, has_prev, L, w);
+        }
+    };
+    // run of the cells beside c (and its own) in the row of cells dy above
+    auto run_of = [&](uint2 c, int dy, uint32_t &b, uint32_t &n) {
+        const int cy = (int)c.y + dy;
+        b = 0;
+        n = 0;
+        if (cy < 0 || cy >= (int)kSparseSide) return;
+        const uint32_t base = (uint32_t)cy * kSparseSide;
+        b = L.start[base + (c.x ? c.x - 1 : 0u)];
+        n = L.start[base + min(c.x + 2, kSparseSide)] - b;
+    };
+    for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        const bool vi = i < cnt;
+        const float2 row = vi ? L.pos[i] : make_float2(0.0f, 0.0f);
+        uint32_t b0 = 0, nb = 0, c0 = 0, nc = 0, g = 0;
+        if (vi) {
+            const uint2 c = cell_of(row);
+            g = off + L.at[i];
+            run_of(c, 0, b0, nb);
+            nb = b0 + nb - (i + 1);   // the rest of the run
+            run_of(c, 1, c0, nc);
+        }
+        scan(row, g, 0u, i + 1, nb, c0, nc, 0u, 0u);
+    }
+    for (uint32_t u0 = 0; u0 < ucnt; u0 += 64) {
+        const uint32_t u = u0 + lane;
+        float2 row = make_float2(0.0f, 0.0f);
+        uint32_t a0 = 0, na = 0, b0 = 0, nb = 0, c0 = 0, nc = 0;
+        if (u < ucnt) {
+            if (u0) ug = reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + u)[3];
+            row = make_float2((float)((tv.sx[ug] - lo.x) * ix), (float)((tv.sy[ug] - lo.y) * iy));
+            const uint2 c = cell_of(row);
+            run_of(c, -1, a0, na);
+            run_of(c, 0, b0, nb);
+            run_of(c, 1, c0, nc);
+        }
+        scan(row, uoff + u, kSparseUnit, a0, na, b0, nb, c0, nc);
+    }
+    if (lane == 0) w.tests += (unsigned long long)cnt * (cnt - 1) / 2 + (unsigned long long)cnt * ucnt;
+}
+
 // Upper-triangle task t of n row blocks -> (r <= q), row-major.
 __device__ __forceinline__ void triangle_task(uint32_t t, uint32_t n, uint32_t &r, uint32_t &q)
 {
@@ -2534,7 +2847,13 @@ __device__ __forceinline__ void triangle_task(uint32_t t, uint32_t n, uint32_t &
 template <int TILE, bool GEO = false, class P>
 __device__ __forceinline__ void join_body(const DevState s, const P blk)
 {
-    __shared__ JoinLds<TILE> lds;
+    __shared__ union {
+        JoinLds<TILE> tiles;
+        SparseLds sparse[kBlock / 64];   // before the first tile
+    } shared;
+    __shared__ JoinSums sums;
+    JoinLds<TILE> &lds = shared.tiles;
+    if (threadIdx.x < kJoinSums) sums.of[threadIdx.x] = 0;   // (barriers follow before their use)
     const double *xy = s.tp->xy;
     const double *xy_prev = s.tp->xy_prev;
     const bool has_prev = s.tp->has_prev != 0;
@@ -2545,7 +2864,6 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = lane_id();
     Stager st{contact_out(s), lds.stage[wave], 0, 0, s.chunk, 0};
     JoinRows &rows = lds.rows[wave];
-    if (threadIdx.x == 0) lds.next = 0;   // (the first leaf's barriers come before any use)
     uint32_t n_in = 0, n_bd = 0;                   // sure contacts (per lane)
     uint32_t pass_in = 0, pass_bd = 0, band = 0;   // band entries within reach / re-tested (per lane)
     uint32_t dups = 0;                             // unstored pairs found twice (per lane)
@@ -2721,7 +3039,41 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
             lds.leaf = L;
         }
     };
-    if (threadIdx.x == 0) fetch_leaf();
+    // The sparse leaves first, one wave each: the queue of tiles after them
+    // evens out what their shares differ by.  The keys that the waves still
+    // hold at the end go out with one reservation.
+    const uint32_t nsp = (s.ctr->error & kErrUnitCap) ? 0 : s.ctr->n_sparse;
+    if (blk.id() * (kBlock / 64) < nsp) {
+        SparseLds &L = shared.sparse[wave];
+        SparseWave w{};
+        for (uint32_t k = blk.id() * (kBlock / 64) + wave; k < nsp; k += blk.count() * (kBlock / 64))
+            join_sparse<GEO>(s, tv, has_prev, L, w, __builtin_amdgcn_readfirstlane(s.sparse_list[k]));
+        while (w.n) sparse_drain<GEO>(s, tv, has_prev, L, w);
+        if (lane == 0) sums.left[wave] = w.nout;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (uint32_t k = 0; k < kBlock / 64; k++) {
+            before += k < wave ? sums.left[k] : 0u;
+            all += sums.left[k];
+        }
+        if (all) {   // (the same in every wave)
+            if (threadIdx.x == 0) sums.base = atomicAdd(&s.ctr->n_clist, (unsigned long long)all);
+            __syncthreads();
+            sparse_write(s, L.out, w.nout, sums.base + before);
+        }
+        st.kept += w.kept;
+        pass_in += w.pass_in;
+        pass_bd += w.pass_bd;
+        band += w.band;
+        dups += w.dups;
+        tests += w.tests;
+        evals += w.evals;
+        __syncthreads();   // the tiles take over the waves' shares of the LDS
+    }
+    if (threadIdx.x == 0) {
+        lds.next = 0;
+        fetch_leaf();
+    }
     __syncthreads();
     for (;;) {
         const uint32_t item = lds.item;
@@ -2797,7 +3149,10 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
         }
     }
     stage_close(st, s);
-    // one atomic per wave for each counter
+    // The workgroup's counts are added up in LDS, then into one of
+    // kJoinParts lines (k_bucket_count adds the lines up): the atomics of a
+    // whole launch on one line run one after another, about 5.5 ns each, and
+    // 4096 waves with five counters each had taken 110 us.
     uint32_t pi_ = pass_in + n_in, pb = pass_bd + n_bd, bd = band, du = dups;
     for (int d = 32; d >= 1; d >>= 1) {
         pi_ += __shfl_xor(pi_, d);
@@ -2807,15 +3162,14 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
     }
     tests = wave_sum_u64(tests);
     if (lane == 0) {
-        const uint32_t ci = pi_, cb = pb;
-        if (tests) atomicAdd(&s.ctr->n_tests, tests);
-        if (evals) atomicAdd(&s.ctr->n_evals, 64ull * evals);
-        if (ci + cb) atomicAdd(&s.ctr->n_contacts, (unsigned long long)(ci + cb));
-        if (cb) atomicAdd(&s.ctr->n_contacts_border, (unsigned long long)cb);
-        if (bd) atomicAdd(&s.ctr->n_rechecks, (unsigned long long)bd);
-        if (st.kept) atomicAdd(&s.ctr->n_stored, (unsigned long long)st.kept);
-        if (du) atomicAdd(&s.ctr->n_dup, (unsigned long long)du);
+        const unsigned long long v[kJoinSums] = {(unsigned long long)pi_ + pb, pb, du, st.kept, bd, tests,
+                                                 64ull * evals};
+        for (uint32_t k = 0; k < kJoinSums; k++)
+            if (v[k]) atomicAdd(&sums.of[k], v[k]);
     }
+    __syncthreads();
+    if (threadIdx.x < kJoinSums && sums.of[threadIdx.x])
+        atomicAdd(&s.jpart[(blk.id() % kJoinParts) * kJoinPartStride + threadIdx.x], sums.of[threadIdx.x]);
 }
 
 template <int TILE, bool GEO = false>
@@ -2856,7 +3210,25 @@ __device__ __forceinline__ void bucket_count_body(const DevState s, const P blk)
 {
     __shared__ uint32_t hist[kMaxCoarse + 1];
     const unsigned long long n = min(s.ctr->n_clist, s.clist_cap);
-    const TableShape sh = table_shape(s);
+    // the join's counts: every workgroup needs those stored, the first leaves
+    // all of them in the counters (a lane per line)
+    static_assert(kJoinParts == 64, "one line per lane");
+    const unsigned long long *part = s.jpart + (size_t)lane_id() * kJoinPartStride;
+    const unsigned long long stored = wave_sum_u64(part[kSumStored]);
+    if (blk.id() == 0 && threadIdx.x < 64) {
+        unsigned long long v[kJoinSums];
+        for (uint32_t k = 0; k < kJoinSums; k++) v[k] = wave_sum_u64(part[k]);
+        if (threadIdx.x == 0) {
+            s.ctr->n_contacts = v[kSumContacts];
+            s.ctr->n_contacts_border = v[kSumBorder];
+            s.ctr->n_dup = v[kSumDup];
+            s.ctr->n_stored = v[kSumStored];
+            s.ctr->n_rechecks = v[kSumBand];
+            s.ctr->n_tests = v[kSumTests];
+            s.ctr->n_evals = v[kSumEvals];
+        }
+    }
+    const TableShape sh = table_shape(s, stored);
     for (uint32_t k = threadIdx.x; k <= sh.coarse; k += kBlock) hist[k] = 0;
     __syncthreads();
     unsigned long long b0, b1;
@@ -3741,7 +4113,7 @@ glint_status build_tree(glint_ctx *c)
     }
     for (int level = 0; level < 64; level++) {
         k_fill_u32<<<gnode, kBlock, 0, c->stream>>>(s.count, 0u, s.node_cap);
-        k_reset_tick<<<1, 1, 0, c->stream>>>(s);
+        k_reset_tick<<<1, kBlock, 0, c->stream>>>(s);
         k_build_count<<<gn, kBlock, 0, c->stream>>>(s);
         k_build_collect<<<gnode, kBlock, 0, c->stream>>>(s);
         glint_status st = read_counters(c);
@@ -3875,7 +4247,7 @@ void enqueue_grid_rebuild(const Seq &q)
 void enqueue_partition(const Seq &q)
 {
     step_fill(q, K_FILL_COUNTS, kFillCount);
-    GLINT_STEP(q, K_RESET, 1, 1u, reset_tick);
+    GLINT_STEP(q, K_RESET, kBlock, 1u, reset_tick);
     if (q.rep().cfg.dynamic_schema == GLINT_SCHEMA_GRID_REBUILD) enqueue_grid_rebuild(q);
     if (q.rep().s.incremental) GLINT_STEP(q, K_REGIONS, kBlock, grid_for(c.s.node_cap), regions);
     GLINT_STEP(q, K_ASSIGN, kBlock, grid_for(c.s.n), assign);
@@ -4273,6 +4645,8 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
         const double u = std::ldexp(1.0, -24);
         double w = (eps / 2 - (2 + std::sqrt(2.0)) * u * (r + eps)) / (2 * std::sqrt(2.0) * u * (1 + u)) - r;
         s.w32_max = w > 0 ? w : 0.0;
+        // beyond what either test accepts (the FP32 one up to 3/2 eps past r)
+        s.guard_reach = cfg->precision == GLINT_PRECISION_FP32_GUARD ? 2 * eps : 0.0;
         s.pf_lim = s.w32_max + r;
     }
 
@@ -4348,6 +4722,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
     ALLOC(s.split_list, node_cap);
     ALLOC(s.merge_list, node_cap);
     ALLOC(s.leaf_list, node_cap);
+    ALLOC(s.sparse_list, node_cap);
     ALLOC(s.sleafb[0], N);
     ALLOC(s.sleafb[1], N);
     ALLOC(s.parent, node_cap);
@@ -4405,6 +4780,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
     }
     ALLOC(s.meet, s.meet_cap);
     ALLOC(s.ctr, 1);
+    ALLOC(s.jpart, (uint64_t)kJoinParts * kJoinPartStride);
     for (int g = 0; g < 2; g++) {
         ALLOC(c->tab[g].keys, s.clist_cap);
         ALLOC(c->tab[g].starts, s.clist_cap);

@@ -97,7 +97,7 @@ struct Counters {
     uint32_t n_drop_leaves;         // leaves over 2*cap this tick (the reference's leaf storage, filter.cpp:100-104)
     uint32_t sorted_valid;          // spid holds a complete leaf order (after the first scatter)
     uint32_t tab_bits;              // log2(regions) of the last tick's table
-    uint32_t pad0_;
+    uint32_t n_sparse;              // leaves joined by one wave each (sparse_list)
     unsigned long long n_drop_objs; // objects beyond 2*cap in those leaves
     unsigned long long n_tests;     // candidate pairs the join tested (the reference's distance tests)
     unsigned long long n_evals;     // pair slots the join evaluated (64 per column of a wave task)
@@ -200,6 +200,7 @@ struct DevState {
     double xbuf, ybuf;  // last_valid margins (filter.cpp:30-31): r, or r in degrees at the root's low latitude
     double *sgeo;       // geography: degrees of longitude per metre at each sorted object's latitude
     double w32_max;     // widest leaf decided in FP32 (error bound inside the band)
+    double guard_reach; // guard mode: width past the reach the sparse join's cells allow for
     double pf_lim;      // largest FP32 offset with the same error bound (w32_max + r)
     unsigned long long unit_cap;
     unsigned long long meet_cap;
@@ -216,6 +217,7 @@ struct DevState {
     uint32_t *split_list;
     uint32_t *merge_list;
     uint32_t *leaf_list;
+    uint32_t *sparse_list;  // leaves the join gives to one wave each
     uint32_t *parent;       // per node: its parent (kNone for the root), for stackless tree walks
     double4 *region;        // per node: the points the descent sends into it, (x.lo, x.hi] x (y.lo, y.hi]
     uint32_t incremental;   // objects are placed from their leaf of the tick before (not with the grid rebuild)
@@ -277,6 +279,7 @@ struct DevState {
     uint32_t heavy_cap;            // fine histograms held
     uint32_t glist_cap;            // branch blocks held per depth
     Counters *ctr;
+    unsigned long long *jpart;     // the join's counts of the tick, in lines of their own
 };
 
 // SplitMix64 finaliser (Steele, Lea, Flood 2014): slot hash of a pair key.
