@@ -56,12 +56,12 @@ struct alignas(64) Node {
 };
 static_assert(sizeof(Node) == 64, "one node per 64-byte line");
 
-// An object whose lookup runs this tick: id, last_valid, leaf and position.
+// An object whose lookup runs this tick: its place in the assignment's order
+// (what the lookup needs of it is read there) and its last_valid, with
+// kBorderOrdered when that place is also its sorted position at the tick before.
+constexpr uint32_t kBorderOrdered = 0x80000000u;   // (node ids stay below)
 struct alignas(8) BorderObj {
-    uint32_t pid, lv, leaf, pleaf;   // pleaf: its leaf at the tick before
-    uint32_t prevk;                  // its sorted position at the tick before (kNone: none known)
-    uint32_t rank;                   // its rank in its leaf (sorted position offset[leaf] + rank)
-    double x, y;
+    uint32_t k, lv;
 };
 
 struct alignas(16) NodeMeta {
@@ -80,7 +80,7 @@ struct Counters {
     unsigned long long n_meet;
     unsigned long long n_rechecks;
     unsigned long long n_clist;     // contact-list entries reserved this tick (chunks)
-    unsigned long long work_border;
+    unsigned long long next_unit;   // units given to leaves (k_scan_units)
     int32_t free_top;
     uint32_t n_split;
     uint32_t n_merge;
@@ -91,7 +91,7 @@ struct Counters {
     uint32_t max_leaf;
     uint32_t error;
     uint32_t work_inside;
-    uint32_t n_nodes;
+    uint32_t next_object;   // places in the sorted arrays given to leaves (k_scan_objects)
     uint32_t last_splits;
     uint32_t last_merges;
     uint32_t n_drop_leaves;         // leaves over 2*cap this tick (the reference's leaf storage, filter.cpp:100-104)
