@@ -82,10 +82,10 @@ def algorithmic_bytes(kernel: str, n: int, per_tick: dict, precision: int) -> fl
         return 8.0 * S
     if kernel == "k_assign":
         return 16.0 * n + 8.0 * n             # xy in, leaf and rank out
-    if kernel == "k_scatter":
-        return 16.0 * n + 8.0 * n + 20.0 * n  # xy, leaf/rank in; sorted xy + id out
-    if kernel == "k_lookup":
-        return 8.0 * per_tick["border_objects"] + 16.0 * per_tick["border_objects"] + 8.0 * U
+    if kernel == "k_place":
+        # the scatter (xy, leaf and rank in; sorted xy and id out) and the lookup (border objects in, units out)
+        return 16.0 * n + 8.0 * n + 20.0 * n + 8.0 * per_tick["border_objects"] + \
+            16.0 * per_tick["border_objects"] + 8.0 * U
     return 0.0
 
 
@@ -146,16 +146,13 @@ def profiled_valu(kernel: str, workload: str, precision: int,
 # lookup, reachability = join and the grouping of contacts by table region,
 # update_meetings = the table update, update_schema); the scans serve all three
 STAGE_OF_KERNEL = {
-    "k_fill_u32": "filter", "k_reset_tick": "filter", "k_regions": "filter", "k_assign": "filter",
-    "k_scan_objects": "filter", "k_scatter": "filter", "k_fill_ucount": "filter", "k_lookup": "filter",
+    "k_begin_tick": "filter", "k_assign": "filter", "k_scan_objects": "filter", "k_place": "filter",
     "k_scan_units": "filter", "k_unit_scatter": "filter", "k_grid_cells": "filter", "k_grid_pyramid": "filter",
     "k_grid_top": "filter", "k_grid_fine_zero": "filter", "k_grid_fine": "filter", "k_grid_level": "filter",
-    "k_join": "reachability", "k_bucket_count": "reachability", "k_scan_write": "reachability",
-    "k_bucket_scatter": "reachability", "k_bucket_fine": "reachability",
-    "k_table": "update_meetings", "k_table_reshaped": "update_meetings", "k_pos32": "update_meetings",
-    "k_log_append": "update_meetings",
-    "k_collect": "update_schema", "k_split": "update_schema", "k_merge": "update_schema",
-    "k_schema_done": "update_schema",
+    "k_join": "reachability", "k_bucket_count": "reachability", "k_scan_reduce": "reachability",
+    "k_scan_top": "reachability", "k_scan_write": "reachability", "k_bucket_scatter": "reachability",
+    "k_bucket_fine": "reachability", "k_table": "update_meetings", "k_pos32": "update_meetings",
+    "k_collect": "update_schema", "k_schema": "update_schema",
 }
 
 

@@ -364,16 +364,7 @@ __device__ __forceinline__ void advance_tick(TickParams *tp, uint64_t stride)
     tp->sy = q;
 }
 
-__global__ void k_advance_tick(TickParams *tp, uint64_t stride) { advance_tick(tp, stride); }
-
-__global__ void kf_advance_tick(const Many m)
-{
-    const Member w = member_of(m);
-    const DevState &s = m.ss[w.i];
-    if (threadIdx.x == 0) advance_tick(s.tp, 2ull * s.n);
-}
-
-// State before the first tick of a run, one k_advance_tick short of it; the
+// State before the first tick of a run, one advance_tick short of it; the
 // positions already point at the first snapshot for the initial build.
 __global__ void k_begin_run(TickParams *tp, const double *base, TableGen tab_old, TableGen tab_cur, float4 *mbr_old,
                             float4 *mbr_cur, double *xy_prev, double *xy_save, uint4 *cand_prev, uint4 *cand,
@@ -408,7 +399,7 @@ __global__ void k_begin_run(TickParams *tp, const double *base, TableGen tab_old
     tp->nstamps = nstamps;
 }
 
-// Tick k of a run is stamped at its start (k_advance_tick, entry 2k) and at
+// Tick k of a run is stamped at its start (advance_tick, entry 2k) and at
 // its end (entry 2k+1), so a tick's latency excludes time spent waiting for
 // other work between ticks.
 __device__ __forceinline__ void stamp_end(TickParams *tp)
@@ -417,16 +408,8 @@ __device__ __forceinline__ void stamp_end(TickParams *tp)
     if (tp->stamps && 2 * k + 1 < tp->nstamps) tp->stamps[2 * k + 1] = wall_clock64();
 }
 
-__global__ void k_stamp(TickParams *tp) { stamp_end(tp); }
-
-__global__ void kf_stamp(const Many m)
-{
-    const Member w = member_of(m);
-    if (threadIdx.x == 0) stamp_end(m.ss[w.i].tp);
-}
-
-template <class P>
-__device__ __forceinline__ void reset_tick_body(const DevState s, const P blk)
+// The tick's counters cleared, by one workgroup.
+__device__ __forceinline__ void reset_tick_body(const DevState &s)
 {
     for (uint32_t k = threadIdx.x; k < kJoinParts * kJoinPartStride; k += blockDim.x) s.jpart[k] = 0;
     if (threadIdx.x != 0) return;
@@ -457,12 +440,7 @@ __device__ __forceinline__ void reset_tick_body(const DevState s, const P blk)
     c->g_heavy = 0;
 }
 
-__global__ void k_reset_tick(DevState s) { reset_tick_body(s, this_blk()); }
-__global__ void kf_reset_tick(const Many m)
-{
-    const Member w = member_of(m);
-    reset_tick_body(m.ss[w.i], w.blk);
-}
+__global__ void k_reset_tick(DevState s) { reset_tick_body(s); }
 
 // ------------------------------------------------------------ tree build
 
@@ -642,13 +620,7 @@ __device__ __forceinline__ void split_body(const DevState s, const P blk, int bu
     }
 }
 
-__global__ void k_split(DevState s, int build_boxes) { split_body(s, this_blk(), build_boxes); }
-__global__ void kf_split(const Many m, int build_boxes)
-{
-    const Member w = member_of(m);
-    split_body(m.ss[w.i], w.blk, build_boxes);
-}
-
+__global__ void k_split(DevState s) { split_body(s, this_blk(), 1); }   // (the initial build)
 // geometry.cu:1166-1190: the four leaf children return to the pool.
 template <class P>
 __device__ __forceinline__ void merge_body(const DevState s, const P blk)
@@ -677,71 +649,66 @@ __device__ __forceinline__ void merge_body(const DevState s, const P blk)
     }
 }
 
-__global__ void k_merge(DevState s) { merge_body(s, this_blk()); }
-__global__ void kf_merge(const Many m)
+// geometry.cu:1193-1234: decisions from this tick's counts, before any
+// change.  Listed by k_scan_objects in a run of ticks, which visits every
+// node's count anyway; by k_collect where the stages are called one by one
+// (the update may then be left out, and must leave no trace of itself).
+__device__ __forceinline__ void collect_node(const DevState &s, uint32_t n, bool in)
 {
-    const Member w = member_of(m);
-    merge_body(m.ss[w.i], w.blk);
-}
-
-// geometry.cu:1193-1234: decisions from this tick's counts, before any change.
-template <class P>
-__device__ __forceinline__ void collect_body(const DevState s, const P blk)
-{
-    for (uint32_t n = blk.id() * blockDim.x + threadIdx.x; n < s.node_cap; n += blk.count() * blockDim.x) {
-        NodeMeta m = s.meta[n];
-        bool split = false, merge = false;
-        if (m.type == kLeaf) {
-            Node nd = s.nodes[n];
-            // height(mbr) > 2r (geometry.cu:1200), height in metres (geometry.cu:30) with geography
-            const double ht = s.geography ? (nd.hy - nd.ly) / kDegPerMeterLat : nd.hy - nd.ly;
-            if (ht > 2 * s.r && s.count[n] > s.cap) {
-                if (++m.overflow >= s.delay) {
-                    split = true;
-                    m.overflow = 0;
-                }
-            } else {
+    NodeMeta m{};
+    if (in) m = s.meta[n];
+    bool split = false, merge = false;
+    if (m.type == kLeaf) {
+        const double2 lo = reinterpret_cast<const double2 *>(s.nodes + n)[1], hi = node_high(s.nodes, n);
+        // height(mbr) > 2r (geometry.cu:1200), height in metres (geometry.cu:30) with geography
+        const double ht = s.geography ? (hi.y - lo.y) / kDegPerMeterLat : hi.y - lo.y;
+        const uint32_t was = m.overflow;
+        if (ht > 2 * s.r && s.count[n] > s.cap) {
+            if (++m.overflow >= s.delay) {
+                split = true;
                 m.overflow = 0;
             }
-            s.meta[n] = m;
-        } else if (m.type == kBranch) {
-            Node nd = s.nodes[n];
-            int leafchild = 0;
-            int ncounter = 0;
-            for (int i = 0; i < 4; i++) {
-                uint32_t c = nd.child[i];
-                if (s.meta[c].type == kLeaf) {
-                    leafchild++;
-                    ncounter += (int)s.count[c];
-                }
+        } else {
+            m.overflow = 0;
+        }
+        if (m.overflow != was) s.meta[n].overflow = m.overflow;
+    } else if (m.type == kBranch) {
+        const uint4 ch = node_children(s.nodes, n);
+        int leafchild = 0;
+        int ncounter = 0;
+        for (int i = 0; i < 4; i++) {
+            const uint32_t c = pick_child(ch, i);
+            if (s.meta[c].type == kLeaf) {
+                leafchild++;
+                ncounter += (int)s.count[c];
             }
-            if (leafchild == 4 && ncounter < (int)s.cap) {
-                if (++m.underflow >= s.delay) {
-                    merge = true;
-                    m.underflow = 0;
-                }
-            } else {
+        }
+        const uint32_t was = m.underflow;
+        if (leafchild == 4 && ncounter < (int)s.cap) {
+            if (++m.underflow >= s.delay) {
+                merge = true;
                 m.underflow = 0;
             }
-            s.meta[n] = m;
+        } else {
+            m.underflow = 0;
         }
-        uint32_t is = wave_append_u32(&s.ctr->n_split, split);
-        if (split) s.split_list[is] = n;
-        uint32_t im = wave_append_u32(&s.ctr->n_merge, merge);
-        if (merge) s.merge_list[im] = n;
+        if (m.underflow != was) s.meta[n].underflow = m.underflow;
     }
+    const uint32_t is = wave_append_u32(&s.ctr->n_split, split);
+    if (split) s.split_list[is] = n;
+    const uint32_t im = wave_append_u32(&s.ctr->n_merge, merge);
+    if (merge) s.merge_list[im] = n;
 }
 
-__global__ void k_collect(DevState s) { collect_body(s, this_blk()); }
-__global__ void kf_collect(const Many m)
+__global__ __launch_bounds__(kBlock) void k_collect(DevState s)
 {
-    const Member w = member_of(m);
-    collect_body(m.ss[w.i], w.blk);
+    const uint32_t stride = gridDim.x * kBlock;
+    for (uint32_t n0 = blockIdx.x * kBlock; n0 < s.node_cap; n0 += stride)
+        collect_node(s, n0 + threadIdx.x, n0 + threadIdx.x < s.node_cap);
 }
 
 // End of a tick: schema change counts and the running totals.
-template <class P>
-__device__ __forceinline__ void schema_done_body(const DevState s, const P blk)
+__device__ __forceinline__ void schema_done(const DevState &s)
 {
     Counters *c = s.ctr;
     c->last_splits = c->n_split;
@@ -769,29 +736,25 @@ __device__ __forceinline__ void schema_done_body(const DevState s, const P blk)
     if (s.mlog) c->n_mlog += c->n_meet < s.meet_cap ? c->n_meet : s.meet_cap;
 }
 
-__global__ void k_schema_done(DevState s) { schema_done_body(s, this_blk()); }
-__global__ void kf_schema_done(const Many m)
+// End of a tick, one workgroup: the listed leaves split, the listed branches
+// merged, the totals advanced and, in a run, the tick stamped.  A tick
+// changes few leaves (about 800 of 80k at 10M objects in hotspots), so the
+// four launches that did this had been waiting, 4.5 us each.
+constexpr int kSchemaThreads = 1024;
+__device__ __forceinline__ void schema_body(const DevState &s, bool run)
 {
-    const Member w = member_of(m);
-    schema_done_body(m.ss[w.i], w.blk);
+    if (threadIdx.x == kSchemaThreads - 1) schema_done(s);   // (beside the splits: it reads counts they leave alone)
+    split_body(s, Blk{0, 1}, 0);
+    __syncthreads();
+    merge_body(s, Blk{0, 1});
+    __syncthreads();
+    if (run && threadIdx.x == 0) stamp_end(s.tp);
 }
 
-// The tick's meetings appended to the meeting log ring (k_schema_done
-// advances its total afterwards).
-template <class P>
-__device__ __forceinline__ void log_append_body(const DevState s, const P blk)
+__global__ __launch_bounds__(kSchemaThreads) void k_schema(DevState s, bool run) { schema_body(s, run); }
+__global__ __launch_bounds__(kSchemaThreads) void kf_schema(const Many m, bool run)
 {
-    const unsigned long long n = min(s.ctr->n_meet, s.meet_cap), base = s.ctr->n_mlog;
-    for (unsigned long long i = blk.id() * (unsigned long long)kBlock + threadIdx.x; i < n;
-         i += (unsigned long long)blk.count() * kBlock)
-        s.mlog[(base + i) % s.mlog_cap] = s.meet[i];
-}
-
-__global__ __launch_bounds__(kBlock) void k_log_append(DevState s) { log_append_body(s, this_blk()); }
-__global__ __launch_bounds__(kBlock) void kf_log_append(const Many m)
-{
-    const Member w = member_of(m);
-    log_append_body(m.ss[w.i], w.blk);
+    schema_body(m.ss[member_of(m).i], run);
 }
 
 // ------------------------------------------------------------ grid rebuild
@@ -821,20 +784,6 @@ constexpr uint32_t kCoarseDepth = 10;
 constexpr uint32_t kCoarseDim = 1u << kCoarseDepth;
 constexpr uint32_t kFineDim = kGridDim / kCoarseDim;       // cells per coarse block side
 constexpr uint32_t kFineCells = kFineDim * kFineDim;
-
-// Per-context arrays cleared by the tick sequence.
-enum FillArray : int { kFillCount, kFillUcount, kFillMeta, kFillCoarse };
-
-template <int F>
-__global__ void kf_fill(const Many m)
-{
-    const Member w = member_of(m);
-    const DevState &s = m.ss[w.i];
-    if (F == kFillCount) fill_body(s.count, 0u, s.node_cap, w.blk);
-    if (F == kFillUcount) fill_body(s.ucount, 0u, s.node_cap, w.blk);
-    if (F == kFillMeta) fill_body(reinterpret_cast<uint32_t *>(s.meta), 0u, 4ull * s.node_cap, w.blk);
-    if (F == kFillCoarse) fill_body(s.g10, 0u, kCoarseDim * kCoarseDim, w.blk);
-}
 
 __host__ __device__ constexpr uint32_t pyr_off(uint32_t d) { return ((1u << (2 * d)) - 1u) / 3u; }
 
@@ -1154,41 +1103,61 @@ __global__ __launch_bounds__(kBlock) void kf_grid_level(const Many m, uint32_t d
 
 // ------------------------------------------------------------ partition
 
-// The region of every node of the tree: the points the descent (child =
+// The region of a node of the tree: the points the descent (child =
 // (y > my)*2 + (x > mx) at every branch) sends into it, the intersection of
 // its ancestors' half-planes, as (x.lo, x.hi] x (y.lo, y.hi] (infinite where
 // no ancestor bounds it).
-template <class P>
-__device__ __forceinline__ void regions_body(const DevState s, const P blk)
+__device__ __forceinline__ void node_region(const DevState &s, uint32_t n)
 {
-    for (uint32_t n = blk.id() * blockDim.x + threadIdx.x; n < s.node_cap; n += blk.count() * blockDim.x) {
-        const int32_t t = s.meta[n].type;
-        if (t != kLeaf && t != kBranch) continue;
-        double xlo = -INFINITY, xhi = INFINITY, ylo = -INFINITY, yhi = INFINITY;
-        for (uint32_t c = n; c != 0;) {
-            const uint32_t a = s.parent[c];
-            const double2 mid = node_mid(s.nodes, a);
-            const uint4 ch = node_children(s.nodes, a);
-            const uint32_t i = ch.x == c ? 0u : ch.y == c ? 1u : ch.z == c ? 2u : 3u;
-            if (i & 1u)
-                xlo = fmax(xlo, mid.x);
-            else
-                xhi = fmin(xhi, mid.x);
-            if (i & 2u)
-                ylo = fmax(ylo, mid.y);
-            else
-                yhi = fmin(yhi, mid.y);
-            c = a;
-        }
-        s.region[n] = make_double4(xlo, xhi, ylo, yhi);
+    const int32_t t = s.meta[n].type;
+    if (t != kLeaf && t != kBranch) return;
+    double xlo = -INFINITY, xhi = INFINITY, ylo = -INFINITY, yhi = INFINITY;
+    for (uint32_t c = n; c != 0;) {
+        const uint32_t a = s.parent[c];
+        const double2 mid = node_mid(s.nodes, a);
+        const uint4 ch = node_children(s.nodes, a);
+        const uint32_t i = ch.x == c ? 0u : ch.y == c ? 1u : ch.z == c ? 2u : 3u;
+        if (i & 1u)
+            xlo = fmax(xlo, mid.x);
+        else
+            xhi = fmin(xhi, mid.x);
+        if (i & 2u)
+            ylo = fmax(ylo, mid.y);
+        else
+            yhi = fmin(yhi, mid.y);
+        c = a;
     }
+    s.region[n] = make_double4(xlo, xhi, ylo, yhi);
 }
 
-__global__ __launch_bounds__(kBlock) void k_regions(DevState s) { regions_body(s, this_blk()); }
-__global__ __launch_bounds__(kBlock) void kf_regions(const Many m)
+// Start of a tick, one launch (five had taken 20 us): the per-node counts and the tick's counters
+// cleared, every node's region (or, for the grid rebuild, the node table and
+// the coarse histogram cleared) and, in a run, the tick advanced.
+template <class P>
+__device__ __forceinline__ void begin_tick_body(const DevState &s, const P blk, bool run)
+{
+    if (blk.id() == 0) {
+        reset_tick_body(s);
+        if (run && threadIdx.x == 0) advance_tick(s.tp, 2ull * s.n);
+    }
+    const uint32_t stride = blk.count() * kBlock, at = blk.id() * kBlock + threadIdx.x;
+    for (uint32_t n = at; n < s.node_cap; n += stride) {
+        s.count[n] = 0;
+        s.ucount[n] = 0;
+        if (s.incremental)
+            node_region(s, n);
+        else
+            s.meta[n] = NodeMeta{};
+    }
+    if (!s.incremental)
+        for (uint32_t k = at; k < kCoarseDim * kCoarseDim; k += stride) s.g10[k] = 0;
+}
+
+__global__ __launch_bounds__(kBlock) void k_begin_tick(DevState s, bool run) { begin_tick_body(s, this_blk(), run); }
+__global__ __launch_bounds__(kBlock) void kf_begin_tick(const Many m, bool run)
 {
     const Member w = member_of(m);
-    regions_body(m.ss[w.i], w.blk);
+    begin_tick_body(m.ss[w.i], w.blk, run);
 }
 
 __device__ __forceinline__ bool in_region(const double4 &r, double x, double y)
@@ -1505,10 +1474,15 @@ __global__ __launch_bounds__(kBlock) void kf_scan_top(const Many m)
 // Object offsets of every leaf and the leaf statistics.  The workgroups take
 // their stretches of the sorted arrays with one atomic each, in any order
 // (only that a leaf's objects are together matters), so there is no pass over
-// the counts before this one.
-template <class P>
+// the counts before this one.  COLLECT: with the schema update's decisions.
+template <bool COLLECT, class P>
 __device__ __forceinline__ void scan_objects_body(const DevState s, const P blk)
 {
+    if constexpr (COLLECT)
+        for (uint32_t k = 0; k < kScanItems; k++) {
+            const uint32_t n = blk.id() * kScanTile + k * kBlock + threadIdx.x;
+            collect_node(s, n, n < s.node_cap);
+        }
     uint32_t base = blk.id() * kScanTile + threadIdx.x * kScanItems;
     uint32_t c[kScanItems];
     uint32_t v = 0;
@@ -1558,11 +1532,13 @@ __device__ __forceinline__ void scan_objects_body(const DevState s, const P blk)
     if (threadIdx.x == 1 && stats[1]) atomicAdd(&s.ctr->n_leaves, stats[1]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_objects(DevState s) { scan_objects_body(s, this_blk()); }
+template <bool COLLECT>
+__global__ __launch_bounds__(kBlock) void k_scan_objects(DevState s) { scan_objects_body<COLLECT>(s, this_blk()); }
+template <bool COLLECT>
 __global__ __launch_bounds__(kBlock) void kf_scan_objects(const Many m)
 {
     const Member w = member_of(m);
-    scan_objects_body(m.ss[w.i], w.blk);
+    scan_objects_body<COLLECT>(m.ss[w.i], w.blk);
 }
 
 // The join's reach in the coordinates of a leaf's box, never less than the
@@ -1588,6 +1564,8 @@ __device__ __forceinline__ double2 sparse_reach(const DevState &s, double ly, do
 template <class P>
 __device__ __forceinline__ void scan_units_body(const DevState s, const P blk)
 {
+    // the scatter before has put the objects in leaf order (read by the next tick)
+    if (blk.id() == 0 && threadIdx.x == 0) s.ctr->sorted_valid = 1;
     uint32_t base = blk.id() * kScanTile + threadIdx.x * kScanItems;
     uint32_t c[kScanItems];
     uint32_t v = 0;
@@ -1691,15 +1669,6 @@ __device__ __forceinline__ void scatter_body(const DevState s, const P blk)
     }
 }
 
-template <bool GEO>
-__global__ __launch_bounds__(kBlock) void k_scatter(DevState s) { scatter_body<GEO>(s, this_blk()); }
-template <bool GEO>
-__global__ __launch_bounds__(kBlock) void kf_scatter(const Many m)
-{
-    const Member w = member_of(m);
-    scatter_body<GEO>(m.ss[w.i], w.blk);
-}
-
 __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t *total)
 {
     uint32_t inc = wave_inclusive_scan(v);
@@ -1792,8 +1761,6 @@ template <bool GEO, class P>
 __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
 {
     const uint32_t nb = s.ctr->n_border;
-    // the scatter before has put the objects in leaf order (read by the next tick)
-    if (blk.id() == 0 && threadIdx.x == 0) s.ctr->sorted_valid = 1;
     __shared__ uint32_t wunits[2][kBlock / 64];
     __shared__ unsigned long long unit_at[2];
     uint32_t turn = 0;
@@ -1869,13 +1836,37 @@ __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
     }
 }
 
+// The scatter and the lookup in one launch: neither needs the other, the
+// lookup waits on chains of node reads and the scatter moves bytes.  A third
+// of the workgroups look up, first in the launch since theirs are the longer
+// waits (alternating them with the scatter's takes 3% longer at 10M objects
+// and in 32 cities).  Together 56 us at 1M uniform objects (48 + 19 apart),
+// 0.85 ms at 10M in hotspots (0.52 + 0.36).
+constexpr uint32_t kPlaceMax = 8192;
+__host__ __device__ inline uint32_t scatter_blocks(uint32_t n)
+{
+    const uint32_t g = (uint32_t)(((uint64_t)n + kBlock - 1) / kBlock);
+    return g < kPlaceMax ? g : kPlaceMax;
+}
+__host__ __device__ inline uint32_t lookup_blocks(uint32_t n) { return (scatter_blocks(n) + 1) / 2; }
+
+template <bool GEO, class P>
+__device__ __forceinline__ void place_body(const DevState &s, const P blk)
+{
+    const uint32_t nl = lookup_blocks(s.n);
+    if (blk.id() < nl)
+        lookup_body<GEO>(s, Blk{blk.id(), nl});
+    else
+        scatter_body<GEO>(s, Blk{blk.id() - nl, blk.count() - nl});
+}
+
 template <bool GEO>
-__global__ __launch_bounds__(kBlock) void k_lookup(DevState s) { lookup_body<GEO>(s, this_blk()); }
+__global__ __launch_bounds__(kBlock) void k_place(DevState s) { place_body<GEO>(s, this_blk()); }
 template <bool GEO>
-__global__ __launch_bounds__(kBlock) void kf_lookup(const Many m)
+__global__ __launch_bounds__(kBlock) void kf_place(const Many m)
 {
     const Member w = member_of(m);
-    lookup_body<GEO>(m.ss[w.i], w.blk);
+    place_body<GEO>(m.ss[w.i], w.blk);
 }
 
 // Units grouped by target leaf: unit_pid[ustart[leaf] + rank] = object, and
@@ -3568,62 +3559,119 @@ struct TableLds {
     uint32_t ho[KV ? kRegion : 1];    // list index of the old entry they continue (kNoSlot: none)
     glint_meeting stage[NT / 64][kMeetStage];
     float4 sbox[KV ? NT / 64 : 1][KV ? kMeetStage : 1];   // the staged meetings' boxes
+    uint32_t staged[NT / 64], logged[NT / 64];            // every wave's staged meetings, and those in the map box
+    unsigned long long meet_at, log_at;                   // the workgroup's places for them
+    uint32_t dups;
 };
 
-// Writes a wave's staged meetings out with one reservation; with the
-// key-value output, those whose box lies in the map box (geometry.cu:665-670,
-// box_contain geometry.cu:53-58) are also logged with their boxes, with one
-// more reservation.
+// Whether staged meeting j of a wave is logged for the key-value output: its
+// box lies in the map box (geometry.cu:665-670, box_contain geometry.cu:53-58).
+__device__ __forceinline__ bool meeting_in_map(const DevState &s, const float4 *sb, uint32_t j, uint32_t nst)
+{
+    if (j >= nst) return false;
+    const float4 bx = sb[j];
+    return bx.x >= s.lx && bx.z <= s.hx && bx.y >= s.ly && bx.w <= s.hy;
+}
+
+__device__ __forceinline__ uint32_t meetings_in_map(const DevState &s, const float4 *sb, uint32_t nst)
+{
+    uint32_t total = 0;
+    for (uint32_t j0 = 0; j0 < nst; j0 += 64)
+        total += (uint32_t)__popcll(__ballot(meeting_in_map(s, sb, j0 + lane_id(), nst)));
+    return total;
+}
+
+// A wave's staged meetings written at place b of the tick's meetings (and of
+// the meeting log ring, whose total the end of the tick advances), those in
+// the map box also at place k of the key-value log.
+template <bool KV>
+__device__ __forceinline__ void table_store(const DevState &s, const glint_meeting *st, const float4 *sb, uint32_t nst,
+                                            unsigned long long b, unsigned long long k)
+{
+    const uint32_t lane = lane_id();
+    for (uint32_t j = lane; j < nst; j += 64) {
+        if (b + j < s.meet_cap) {
+            s.meet[b + j] = st[j];
+            if (s.mlog) s.mlog[(s.ctr->n_mlog + b + j) % s.mlog_cap] = st[j];
+        } else {
+            atomicOr(&s.ctr->error, kErrMeetCap);
+        }
+    }
+    if constexpr (KV) {
+        for (uint32_t j0 = 0; j0 < nst; j0 += 64) {
+            const uint32_t j = j0 + lane;
+            const bool put = meeting_in_map(s, sb, j, nst);
+            const unsigned long long m = __ballot(put);
+            if (put) {
+                const unsigned long long at = k + __popcll(m & ((1ull << lane) - 1ull));
+                if (at < s.kvlog_cap) {
+                    KvLogEntry e;
+                    e.pid_a = st[j].pid_a;
+                    e.pid_b = st[j].pid_b;
+                    e.start = st[j].start;
+                    e.end = st[j].end;
+                    e.box = sb[j];
+                    s.kvlog[at] = e;
+                } else {
+                    atomicOr(&s.ctr->error, kErrKvCap);
+                }
+            }
+            k += (unsigned long long)__popcll(m);
+        }
+    }
+}
+
+// A wave whose stage is full writes its meetings out alone.
 template <bool KV, int NT>
 __device__ __forceinline__ void table_flush_stage(const DevState &s, glint_meeting *st, const float4 *sb,
                                                   uint32_t &nst)
 {
     wave_sync();
     const uint32_t lane = lane_id();
-    unsigned long long b = 0;
+    unsigned long long b = 0, k = 0;
     if (lane == 0) b = atomicAdd(&s.ctr->n_meet, (unsigned long long)nst);
-    b = __shfl(b, 0);
-    for (uint32_t j = lane; j < nst; j += 64) {
-        if (b + j < s.meet_cap)
-            s.meet[b + j] = st[j];
-        else
-            atomicOr(&s.ctr->error, kErrMeetCap);
+    if constexpr (KV) {
+        const uint32_t logged = meetings_in_map(s, sb, nst);
+        if (lane == 0 && logged) k = atomicAdd(&s.ctr->n_kvlog, (unsigned long long)logged);
+        k = __shfl(k, 0);
+    }
+    table_store<KV>(s, st, sb, nst, __shfl(b, 0), k);
+    wave_sync();
+    nst = 0;
+}
+
+// The staged meetings of all the workgroup's waves, with one reservation: at
+// 10M objects in hotspots (2.6M meetings) the waves had made 60 thousand on
+// one counter, 5.5 ns apart (k_table 1.19 -> 1.07 ms; 253 -> 160 us for 2M
+// objects with the grid rebuild).
+// Every thread calls it, after a barrier behind the waves' L.staged.
+template <bool KV, int NT>
+__device__ __forceinline__ void table_flush_group(const DevState &s, TableLds<KV, NT> &L, const glint_meeting *st,
+                                                  const float4 *sb, uint32_t &nst)
+{
+    const uint32_t wave = threadIdx.x / 64;
+    uint32_t before = 0, all = 0;
+    for (uint32_t w = 0; w < NT / 64; w++) {
+        before += w < wave ? L.staged[w] : 0u;
+        all += L.staged[w];
     }
     if constexpr (KV) {
-        auto in_map = [&](uint32_t j) {
-            if (j >= nst) return false;
-            const float4 bx = sb[j];
-            return bx.x >= s.lx && bx.z <= s.hx && bx.y >= s.ly && bx.w <= s.hy;
-        };
-        uint32_t total = 0;
-        for (uint32_t j0 = 0; j0 < nst; j0 += 64) total += (uint32_t)__popcll(__ballot(in_map(j0 + lane)));
-        if (total) {
-            unsigned long long k = 0;
-            if (lane == 0) k = atomicAdd(&s.ctr->n_kvlog, (unsigned long long)total);
-            k = __shfl(k, 0);
-            for (uint32_t j0 = 0; j0 < nst; j0 += 64) {
-                const uint32_t j = j0 + lane;
-                const bool put = in_map(j);
-                const unsigned long long m = __ballot(put);
-                if (put) {
-                    const unsigned long long at = k + __popcll(m & ((1ull << lane) - 1ull));
-                    if (at < s.kvlog_cap) {
-                        KvLogEntry e;
-                        e.pid_a = st[j].pid_a;
-                        e.pid_b = st[j].pid_b;
-                        e.start = st[j].start;
-                        e.end = st[j].end;
-                        e.box = sb[j];
-                        s.kvlog[at] = e;
-                    } else {
-                        atomicOr(&s.ctr->error, kErrKvCap);
-                    }
-                }
-                k += (unsigned long long)__popcll(m);
-            }
-        }
+        const uint32_t logged = meetings_in_map(s, sb, nst);
+        if (lane_id() == 0) L.logged[wave] = logged;
     }
-    wave_sync();
+    if (threadIdx.x == 0) L.meet_at = atomicAdd(&s.ctr->n_meet, (unsigned long long)all);
+    lds_barrier();
+    uint32_t lbefore = 0;
+    if constexpr (KV) {
+        uint32_t lall = 0;
+        for (uint32_t w = 0; w < NT / 64; w++) {
+            lbefore += w < wave ? L.logged[w] : 0u;
+            lall += L.logged[w];
+        }
+        if (threadIdx.x == 0 && lall) L.log_at = atomicAdd(&s.ctr->n_kvlog, (unsigned long long)lall);
+        lds_barrier();
+    }
+    table_store<KV>(s, st, sb, nst, L.meet_at + before, L.log_at + lbefore);
     nst = 0;
 }
 
@@ -3756,11 +3804,7 @@ __device__ __forceinline__ void table_write(const TableLds<KV, NT> &L, const Dev
 // does not depend on the order of the updates.  Boxes stay in HBM beside the
 // list entries; the points come from a float copy of the positions that
 // fits the last-level cache.
-// RESHAPED: the variant for a tick whose table shape differs from the
-// previous generation's; the host launches both variants and the one that
-// does not apply returns at once (the common variant then needs no registers
-// for the mapping between shapes).
-template <bool KV, int NT, bool RESHAPED, class P>
+template <bool KV, int NT, class P>
 __device__ __forceinline__ void table_body(const DevState s, const P blk)
 {
     __shared__ TableLds<KV, NT> L;
@@ -3771,9 +3815,8 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
     // in its high `bits` bits, so an old region of fewer bits holds the
     // pairs of 2^(bits - pbits) regions (filtered here by the hash), and a
     // region of this tick holds those of 2^(pbits - bits) consecutive old ones
-    const uint32_t bits = table_shape(s).bits, pbits_gen = told.rstart[s.rs_total + 1];
-    if ((pbits_gen != bits) != RESHAPED) return;
-    const uint32_t pbits = RESHAPED ? pbits_gen : bits;
+    const uint32_t bits = __builtin_amdgcn_readfirstlane(table_shape(s).bits);
+    const uint32_t pbits = __builtin_amdgcn_readfirstlane(told.rstart[s.rs_total + 1]);
     const uint32_t nreg = 1u << bits;
     const bool filter_old = pbits < bits;
     // old region range of region rr: rstart[(rr >> dn) << up] .. rstart[((rr >> dn) + 1) << up]
@@ -3813,8 +3856,10 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
             nkn[q] = c < c1n ? tcur.keys[c] : 0ull;
         }
     };
+    if (blk.id() >= nreg) return;
+    if (threadIdx.x == 0) L.dups = 0;   // (the regions' barriers come before its use)
     bounds(blk.id());
-    if (blk.id() < nreg) prefetch(blk.id());
+    prefetch(blk.id());
     for (uint32_t r = blk.id(); r < nreg; r += blk.count()) {
         for (uint32_t k = threadIdx.x; k < kRegion; k += NT) L.hk[k] = kEmptyKey;
         const uint32_t c0 = c0n, c1 = c1n;
@@ -3843,19 +3888,12 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
         }
         lds_barrier();
         // the previous generation's entries of the region
-        if (filter_old) {   // a table that grew since the previous tick: only this region's pairs
+        // (filter_old: a table that grew since the previous tick, only this region's pairs)
 #pragma unroll
-            for (int q = 0; q < kPer; q++) {
-                const uint32_t i = o0 + threadIdx.x + q * NT;
-                const bool mine = region_of(pk[q] & kKeyBits, bits) == r;
-                table_old(L, s, i < o1 && mine, pk[q], ps[q], i, tick, last, st, sb, nst, bits);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < kPer; q++) {
-                const uint32_t i = o0 + threadIdx.x + q * NT;
-                table_old(L, s, i < o1, pk[q], ps[q], i, tick, last, st, sb, nst, bits);
-            }
+        for (int q = 0; q < kPer; q++) {
+            const uint32_t i = o0 + threadIdx.x + q * NT;
+            const bool mine = !filter_old || region_of(pk[q] & kKeyBits, bits) == r;
+            table_old(L, s, i < o1 && mine, pk[q], ps[q], i, tick, last, st, sb, nst, bits);
         }
         for (uint32_t b = o0 + kRegion; b < o1; b += NT) {   // regions of more than kRegion entries
             const uint32_t i = b + threadIdx.x;
@@ -3872,6 +3910,7 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
             const uint32_t c = c0 + threadIdx.x + q * NT;
             if (c < c1 && ns[q] != kNoSlot - 1) table_write(L, s, tcur, nk[q], c, ns[q], tick, last, pp[q]);
         }
+        if (lane_id() == 0) L.staged[threadIdx.x / 64] = nst;
         for (uint32_t c = c0 + kRegion + threadIdx.x; c < c1; c += NT) {
             const unsigned long long k = tcur.keys[c];
             uint32_t q = kNoSlot;
@@ -3882,20 +3921,30 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
             table_write(L, s, tcur, k, c, q, tick, last, pair_pos<KV>(s, k));
         }
         lds_barrier();
+        // the waves' meetings go out together at the end, or before a stage is full
+        uint32_t most = 0, any = 0;
+        for (uint32_t w = 0; w < NT / 64; w++) {
+            most = max(most, L.staged[w]);
+            any |= L.staged[w];
+        }
+        if (most > kMeetStage / 4 || (rn >= nreg && any)) table_flush_group<KV, NT>(s, L, st, sb, nst);
     }
-    if (nst) table_flush_stage<KV, NT>(s, st, sb, nst);
     // distinct pairs of the tick: contacts less second copies
     for (int d = 32; d >= 1; d >>= 1) dups += __shfl_xor(dups, d);
-    if (lane_id() == 0 && dups) atomicAdd(&s.ctr->n_dup, (unsigned long long)dups);
+    if (lane_id() == 0 && dups) atomicAdd(&L.dups, dups);
+    lds_barrier();
+    if (threadIdx.x == 0 && L.dups) atomicAdd(&s.ctr->n_dup, (unsigned long long)L.dups);
 }
 
-template <bool KV, int NT, bool RESHAPED>
-__global__ __launch_bounds__(NT) void k_table(DevState s) { table_body<KV, NT, RESHAPED>(s, this_blk()); }
-template <bool KV, int NT, bool RESHAPED>
+// (as many waves per SIMD as the workgroups that fit a CU's LDS have)
+constexpr int table_waves(bool kv, int nt) { return nt == 256 ? 1 : kv ? 4 : nt == 512 ? 6 : 8; }
+template <bool KV, int NT>
+__global__ __launch_bounds__(NT, table_waves(KV, NT)) void k_table(DevState s) { table_body<KV, NT>(s, this_blk()); }
+template <bool KV, int NT>
 __global__ __launch_bounds__(NT) void kf_table(const Many m)
 {
     const Member w = member_of(m);
-    table_body<KV, NT, RESHAPED>(m.ss[w.i], w.blk);
+    table_body<KV, NT>(m.ss[w.i], w.blk);
 }
 
 // ------------------------------------------------------------ host side
@@ -3931,17 +3980,15 @@ double sqrt_threshold(double r)
 }
 
 enum KernelId {
-    K_FILL_COUNTS, K_RESET, K_ASSIGN, K_SCAN_REDUCE, K_SCAN_TOP, K_SCAN_OBJECTS, K_SCATTER, K_FILL_UCOUNT,
-    K_LOOKUP, K_SCAN_UNITS, K_UNIT_SCATTER, K_JOIN, K_BUCKET_COUNT, K_SCAN_WRITE, K_BUCKET_SCATTER, K_BUCKET_FINE,
-    K_TABLE, K_TABLE_RESHAPED, K_COLLECT, K_SPLIT, K_MERGE, K_SCHEMA_DONE, K_TICK_PARAMS, K_POS32, K_LOG_APPEND, K_GRID_CELLS,
-    K_GRID_PYRAMID, K_GRID_TOP, K_GRID_FINE_ZERO, K_GRID_FINE, K_GRID_LEVEL, K_REGIONS, K_COUNT
+    K_BEGIN_TICK, K_ASSIGN, K_SCAN_OBJECTS, K_PLACE, K_SCAN_UNITS, K_UNIT_SCATTER, K_JOIN, K_BUCKET_COUNT,
+    K_SCAN_REDUCE, K_SCAN_TOP, K_SCAN_WRITE, K_BUCKET_SCATTER, K_BUCKET_FINE, K_POS32, K_TABLE, K_COLLECT, K_SCHEMA,
+    K_GRID_CELLS, K_GRID_PYRAMID, K_GRID_TOP, K_GRID_FINE_ZERO, K_GRID_FINE, K_GRID_LEVEL, K_COUNT
 };
 const char *const kKernelNames[K_COUNT] = {
-    "k_fill_u32", "k_reset_tick", "k_assign", "k_scan_reduce", "k_scan_top", "k_scan_objects", "k_scatter",
-    "k_fill_ucount", "k_lookup", "k_scan_units", "k_unit_scatter", "k_join", "k_bucket_count", "k_scan_write",
-    "k_bucket_scatter", "k_bucket_fine", "k_table", "k_table_reshaped", "k_collect", "k_split", "k_merge", "k_schema_done",
-    "k_advance_tick", "k_pos32", "k_log_append", "k_grid_cells", "k_grid_pyramid", "k_grid_top",
-    "k_grid_fine_zero", "k_grid_fine", "k_grid_level", "k_regions"};
+    "k_begin_tick", "k_assign", "k_scan_objects", "k_place", "k_scan_units", "k_unit_scatter", "k_join",
+    "k_bucket_count", "k_scan_reduce", "k_scan_top", "k_scan_write", "k_bucket_scatter", "k_bucket_fine", "k_pos32",
+    "k_table", "k_collect", "k_schema", "k_grid_cells", "k_grid_pyramid", "k_grid_top", "k_grid_fine_zero",
+    "k_grid_fine", "k_grid_level"};
 
 // Per-kernel HIP-event timing on the context's stream (optional).
 struct KernelProfiler {
@@ -4175,7 +4222,7 @@ glint_status build_tree(glint_ctx *c)
         if (st) return st;
         if (c->h_ctr->error) return status_from_flags(c, c->h_ctr->error);
         if (c->h_ctr->n_split == 0) break;
-        k_split<<<grid_for(c->h_ctr->n_split), kBlock, 0, c->stream>>>(s, 1);
+        k_split<<<grid_for(c->h_ctr->n_split), kBlock, 0, c->stream>>>(s);
     }
     HIP_TRY(c, hipGetLastError());
     c->built = true;
@@ -4197,6 +4244,7 @@ struct FusedGroup {
 struct Seq {
     glint_ctx *one = nullptr;
     const FusedGroup *group = nullptr;
+    bool run = false;   // a tick of a run: advanced on the device, every stage follows
     const glint_ctx &rep() const { return one ? *one : *group->ctx[0]; }
 };
 
@@ -4231,31 +4279,7 @@ void step(const Seq &q, int id, B blocks, S single, F fused)
         [&](hipStream_t st_, uint32_t g_, glint_ctx &c) { k_##name<<<g_, threads, 0, st_>>>(c.s); },     \
         [&](hipStream_t st_, uint32_t g_, const Many &m_) { kf_##name<<<g_, threads, 0, st_>>>(m_); })
 
-// Clearing of a per-node counter array.
-void step_fill(const Seq &q, int id, int which)
-{
-    step(
-        q, id,
-        [&](const glint_ctx &c) -> uint32_t {
-            return which == kFillCoarse ? grid_for(kCoarseDim * kCoarseDim)
-                                        : grid_for((which == kFillMeta ? 4ull : 1ull) * c.s.node_cap);
-        },
-        [&](hipStream_t st, uint32_t g, glint_ctx &c) {
-            const DevState &s = c.s;
-            if (which == kFillCount) k_fill_u32<<<g, kBlock, 0, st>>>(s.count, 0u, s.node_cap);
-            if (which == kFillUcount) k_fill_u32<<<g, kBlock, 0, st>>>(s.ucount, 0u, s.node_cap);
-            if (which == kFillMeta)
-                k_fill_u32<<<g, kBlock, 0, st>>>(reinterpret_cast<uint32_t *>(s.meta), 0u, 4ull * s.node_cap);
-            if (which == kFillCoarse) k_fill_u32<<<g, kBlock, 0, st>>>(s.g10, 0u, kCoarseDim * kCoarseDim);
-        },
-        [&](hipStream_t st, uint32_t g, const Many &m) {
-            if (which == kFillCount) kf_fill<kFillCount><<<g, kBlock, 0, st>>>(m);
-            if (which == kFillUcount) kf_fill<kFillUcount><<<g, kBlock, 0, st>>>(m);
-            if (which == kFillMeta) kf_fill<kFillMeta><<<g, kBlock, 0, st>>>(m);
-            if (which == kFillCoarse) kf_fill<kFillCoarse><<<g, kBlock, 0, st>>>(m);
-        });
-}
-
+// The three kernels that scan the region bins.
 void step_scan_bins(const Seq &q)
 {
     auto nb = [](const glint_ctx &c) -> uint32_t { return scan_blocks_for(bins_length(c.s)); };
@@ -4281,8 +4305,6 @@ void step_scan_bins(const Seq &q)
 // assignment: a fixed sequence of launches.
 void enqueue_grid_rebuild(const Seq &q)
 {
-    step_fill(q, K_FILL_COUNTS, kFillCoarse);
-    step_fill(q, K_FILL_COUNTS, kFillMeta);
     GLINT_STEP(q, K_GRID_CELLS, kBlock, grid_for(c.s.n), grid_cells);
     GLINT_STEP(q, K_GRID_PYRAMID, kBlock, 1024u, grid_pyramid);
     GLINT_STEP(q, K_GRID_TOP, 1024, 1u, grid_top);
@@ -4300,25 +4322,29 @@ void enqueue_grid_rebuild(const Seq &q)
 
 void enqueue_partition(const Seq &q)
 {
-    step_fill(q, K_FILL_COUNTS, kFillCount);
-    GLINT_STEP(q, K_RESET, kBlock, 1u, reset_tick);
-    if (q.rep().cfg.dynamic_schema == GLINT_SCHEMA_GRID_REBUILD) enqueue_grid_rebuild(q);
-    if (q.rep().s.incremental) GLINT_STEP(q, K_REGIONS, kBlock, grid_for(c.s.node_cap), regions);
+    step(
+        q, K_BEGIN_TICK,
+        [](const glint_ctx &c) -> uint32_t {
+            return grid_for(std::max<uint64_t>(c.s.node_cap, c.s.incremental ? 0 : kCoarseDim * kCoarseDim));
+        },
+        [&](hipStream_t st, uint32_t g, glint_ctx &c) { k_begin_tick<<<g, kBlock, 0, st>>>(c.s, q.run); },
+        [&](hipStream_t st, uint32_t g, const Many &m) { kf_begin_tick<<<g, kBlock, 0, st>>>(m, q.run); });
+    const uint32_t schema = q.rep().cfg.dynamic_schema;
+    if (schema == GLINT_SCHEMA_GRID_REBUILD) enqueue_grid_rebuild(q);
     GLINT_STEP(q, K_ASSIGN, kBlock, grid_for(c.s.n), assign);
-    GLINT_STEP(q, K_SCAN_OBJECTS, kBlock, c.scan_blocks, scan_objects);
-    if (q.rep().s.geography)
-        GLINT_STEP(q, K_SCATTER, kBlock, grid_for(c.s.n), scatter<true>);
+    if (schema == GLINT_SCHEMA_DYNAMIC && q.run)
+        GLINT_STEP(q, K_SCAN_OBJECTS, kBlock, c.scan_blocks, scan_objects<true>);
     else
-        GLINT_STEP(q, K_SCATTER, kBlock, grid_for(c.s.n), scatter<false>);
+        GLINT_STEP(q, K_SCAN_OBJECTS, kBlock, c.scan_blocks, scan_objects<false>);
 }
 
-void enqueue_lookup(const Seq &q)
+// The objects put in leaf order, the border units found and grouped.
+void enqueue_place(const Seq &q)
 {
-    step_fill(q, K_FILL_UCOUNT, kFillUcount);
     if (q.rep().s.geography)
-        GLINT_STEP(q, K_LOOKUP, kBlock, grid_for(c.s.n), lookup<true>);
+        GLINT_STEP(q, K_PLACE, kBlock, scatter_blocks(c.s.n) + lookup_blocks(c.s.n), place<true>);
     else
-        GLINT_STEP(q, K_LOOKUP, kBlock, grid_for(c.s.n), lookup<false>);
+        GLINT_STEP(q, K_PLACE, kBlock, scatter_blocks(c.s.n) + lookup_blocks(c.s.n), place<false>);
     GLINT_STEP(q, K_SCAN_UNITS, kBlock, c.scan_blocks, scan_units);
     GLINT_STEP(q, K_UNIT_SCATTER, kBlock, grid_for(c.s.unit_cap), unit_scatter);
 }
@@ -4385,19 +4411,12 @@ __global__ __launch_bounds__(kBlock) void kf_pos32(const Many m)
 }
 
 template <bool KV, int NT>
-void step_table(const Seq &q, bool reshaped)
+void step_table(const Seq &q)
 {
-    auto g = [](const glint_ctx &c) -> uint32_t { return c.table_grid; };
-    if (reshaped)
-        step(
-            q, K_TABLE_RESHAPED, g,
-            [&](hipStream_t st, uint32_t n, glint_ctx &c) { k_table<KV, NT, true><<<n, NT, 0, st>>>(c.s); },
-            [&](hipStream_t st, uint32_t n, const Many &m) { kf_table<KV, NT, true><<<n, NT, 0, st>>>(m); });
-    else
-        step(
-            q, K_TABLE, g,
-            [&](hipStream_t st, uint32_t n, glint_ctx &c) { k_table<KV, NT, false><<<n, NT, 0, st>>>(c.s); },
-            [&](hipStream_t st, uint32_t n, const Many &m) { kf_table<KV, NT, false><<<n, NT, 0, st>>>(m); });
+    step(
+        q, K_TABLE, [](const glint_ctx &c) -> uint32_t { return c.table_grid; },
+        [&](hipStream_t st, uint32_t n, glint_ctx &c) { k_table<KV, NT><<<n, NT, 0, st>>>(c.s); },
+        [&](hipStream_t st, uint32_t n, const Many &m) { kf_table<KV, NT><<<n, NT, 0, st>>>(m); });
 }
 
 void enqueue_evaluate(const Seq &q)
@@ -4406,36 +4425,23 @@ void enqueue_evaluate(const Seq &q)
     if (r.kv) GLINT_STEP(q, K_POS32, kBlock, grid_for(c.s.n), pos32);
     // persistent over the regions
     const uint32_t nt = r.cfg.table_threads ? r.cfg.table_threads : 512;
-    // both shape variants; the one that does not apply to the tick returns at once
-    for (int reshaped = 0; reshaped < 2; reshaped++) {
-        if (r.kv)
-            nt == 1024 ? step_table<true, 1024>(q, reshaped) : nt == 512 ? step_table<true, 512>(q, reshaped)
-                                                                         : step_table<true, 256>(q, reshaped);
-        else
-            nt == 1024 ? step_table<false, 1024>(q, reshaped) : nt == 512 ? step_table<false, 512>(q, reshaped)
-                                                                          : step_table<false, 256>(q, reshaped);
-    }
-    GLINT_STEP(q, K_LOG_APPEND, kBlock, c.s.mlog ? 1024u : 0u, log_append);
+    if (r.kv)
+        nt == 1024 ? step_table<true, 1024>(q) : nt == 512 ? step_table<true, 512>(q) : step_table<true, 256>(q);
+    else
+        nt == 1024 ? step_table<false, 1024>(q) : nt == 512 ? step_table<false, 512>(q) : step_table<false, 256>(q);
 }
 
 void enqueue_schema(const Seq &q)
 {
-    if (q.rep().cfg.dynamic_schema == GLINT_SCHEMA_DYNAMIC) {
-        GLINT_STEP(q, K_COLLECT, kBlock, grid_for(c.s.node_cap), collect);
-        step(
-            q, K_SPLIT, [](const glint_ctx &c) -> uint32_t { return grid_for(c.s.node_cap); },
-            [&](hipStream_t st, uint32_t g, glint_ctx &c) { k_split<<<g, kBlock, 0, st>>>(c.s, 0); },
-            [&](hipStream_t st, uint32_t g, const Many &m) { kf_split<<<g, kBlock, 0, st>>>(m, 0); });
-        GLINT_STEP(q, K_MERGE, kBlock, grid_for(c.s.node_cap), merge);
-    }
-    GLINT_STEP(q, K_SCHEMA_DONE, 1, 1u, schema_done);
+    if (q.rep().cfg.dynamic_schema == GLINT_SCHEMA_DYNAMIC && !q.run)   // (a run's ticks: k_scan_objects)
+        launch(q.one, K_COLLECT, [&] {
+            k_collect<<<grid_for(q.one->s.node_cap), kBlock, 0, q.one->stream>>>(q.one->s);
+        });
+    step(
+        q, K_SCHEMA, [](const glint_ctx &) -> uint32_t { return 1; },
+        [&](hipStream_t st, uint32_t g, glint_ctx &c) { k_schema<<<g, kSchemaThreads, 0, st>>>(c.s, q.run); },
+        [&](hipStream_t st, uint32_t g, const Many &m) { kf_schema<<<g, kSchemaThreads, 0, st>>>(m, q.run); });
 }
-
-void enqueue_partition(glint_ctx *c) { enqueue_partition(Seq{c, nullptr}); }
-void enqueue_lookup(glint_ctx *c) { enqueue_lookup(Seq{c, nullptr}); }
-void enqueue_refine(glint_ctx *c) { enqueue_refine(Seq{c, nullptr}); }
-void enqueue_evaluate(glint_ctx *c) { enqueue_evaluate(Seq{c, nullptr}); }
-void enqueue_schema(glint_ctx *c) { enqueue_schema(Seq{c, nullptr}); }
 
 void fill_stats(glint_ctx *c)
 {
@@ -4991,9 +4997,9 @@ glint_status glint_partition(glint_ctx *c)
         if (st) return st;
     }
     HIP_TRY(c, hipEventRecord(c->ev[0], c->stream));
-    enqueue_partition(c);
+    enqueue_partition(Seq{c});
     HIP_TRY(c, hipEventRecord(c->ev[1], c->stream));
-    enqueue_lookup(c);
+    enqueue_place(Seq{c});
     HIP_TRY(c, hipEventRecord(c->ev[2], c->stream));
     HIP_TRY(c, hipGetLastError());
     c->partitioned = true;
@@ -5013,7 +5019,7 @@ glint_status glint_refine(glint_ctx *c)
         return GLINT_ERR_INJECTED;
     }
     HIP_TRY(c, hipSetDevice(c->device));
-    enqueue_refine(c);
+    enqueue_refine(Seq{c});
     HIP_TRY(c, hipEventRecord(c->ev[3], c->stream));
     HIP_TRY(c, hipGetLastError());
     c->refined = true;
@@ -5033,7 +5039,7 @@ glint_status glint_evaluate(glint_ctx *c, glint_meeting *out, uint64_t cap, uint
         return GLINT_ERR_INJECTED;
     }
     HIP_TRY(c, hipSetDevice(c->device));
-    enqueue_evaluate(c);
+    enqueue_evaluate(Seq{c});
     HIP_TRY(c, hipEventRecord(c->ev[4], c->stream));
     HIP_TRY(c, hipGetLastError());
     c->evaluated = true;
@@ -5075,7 +5081,7 @@ glint_status glint_update_schema(glint_ctx *c)
         return GLINT_ERR_INJECTED;
     }
     HIP_TRY(c, hipSetDevice(c->device));
-    enqueue_schema(c);
+    enqueue_schema(Seq{c});
     HIP_TRY(c, hipEventRecord(c->ev[5], c->stream));
     HIP_TRY(c, hipGetLastError());
     return GLINT_OK;
@@ -5091,34 +5097,17 @@ glint_status glint_process_tick(glint_ctx *c, const double *xy, uint32_t tick)
     return glint_update_schema(c);
 }
 
-static void enqueue_tick_body(glint_ctx *c, uint64_t stride)
+// One tick of a run.
+static void enqueue_tick(const Seq &q)
 {
-    launch(c, K_TICK_PARAMS, [&] { k_advance_tick<<<1, 1, 0, c->stream>>>(c->s.tp, stride); });
-    enqueue_partition(c);
-    enqueue_lookup(c);
-    enqueue_refine(c);
-    enqueue_evaluate(c);
-    enqueue_schema(c);
-    k_stamp<<<1, 1, 0, c->stream>>>(c->s.tp);
-}
-
-// One tick of every member of a fused group: one launch per step.
-static void enqueue_tick_body(const FusedGroup &g)
-{
-    const Seq q{nullptr, &g};
-    const uint32_t n = (uint32_t)g.ctx.size();
-    Many m{};
-    m.ss = g.d_states;
-    m.n = n;
-    for (uint32_t i = 0; i <= n; i++) m.start[i] = i;   // one workgroup each
-    kf_advance_tick<<<n, 1, 0, g.stream>>>(m);
     enqueue_partition(q);
-    enqueue_lookup(q);
+    enqueue_place(q);
     enqueue_refine(q);
     enqueue_evaluate(q);
     enqueue_schema(q);
-    kf_stamp<<<n, 1, 0, g.stream>>>(m);
 }
+static void enqueue_tick(glint_ctx *c) { enqueue_tick(Seq{c, nullptr, true}); }
+static void enqueue_tick(const FusedGroup &g) { enqueue_tick(Seq{nullptr, &g, true}); }
 
 // The settings that pick kernel variants; contexts alike in all of them can
 // share fused launches.
@@ -5201,7 +5190,6 @@ glint_status glint_run_ticks(glint_ctx *c, const double *d_trace, uint32_t first
     if (!c || !d_trace || nticks == 0) return GLINT_ERR_INVALID_ARGUMENT;
     glint_status st = run_begin(c, d_trace, first_tick, nticks);
     if (st) return st;
-    const uint64_t stride = 2ull * c->s.n;
     const uint32_t G = c->cfg.graph_ticks;
     uint32_t done = 0;
     if (G && !c->prof.on && nticks >= G) {
@@ -5211,7 +5199,7 @@ glint_status glint_run_ticks(glint_ctx *c, const double *d_trace, uint32_t first
             // exit after the capture began ends it, so the stream stays usable.
             hipGraph_t graph = nullptr;
             HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            for (uint32_t k = 0; k < G; k++) enqueue_tick_body(c, stride);
+            for (uint32_t k = 0; k < G; k++) enqueue_tick(c);
             hipError_t e = hipGetLastError();
             const hipError_t ee = hipStreamEndCapture(c->stream, &graph);
             if (e == hipSuccess) e = ee;
@@ -5224,7 +5212,7 @@ glint_status glint_run_ticks(glint_ctx *c, const double *d_trace, uint32_t first
         }
         for (; done + G <= nticks; done += G) HIP_TRY(c, hipGraphLaunch(c->graph_exec, c->stream));
     }
-    for (; done < nticks; done++) enqueue_tick_body(c, stride);
+    for (; done < nticks; done++) enqueue_tick(c);
     HIP_TRY(c, hipGetLastError());
     run_end_state(c, first_tick, nticks);
     return run_finish(c, nticks, tick_ms);
@@ -5251,8 +5239,7 @@ glint_status glint_run_ticks_noalloc(glint_ctx *c, const double *d_trace, uint32
     float *ms = reinterpret_cast<float *>(stamps + 2 * kNoAllocMaxTicks);
     glint_status st = run_begin(c, d_trace, first_tick, nticks, stamps);
     if (st) return st;
-    const uint64_t stride = 2ull * c->s.n;
-    for (uint32_t k = 0; k < nticks; k++) enqueue_tick_body(c, stride);   // plain launches, no graph
+    for (uint32_t k = 0; k < nticks; k++) enqueue_tick(c);   // plain launches, no graph
     HIP_TRY(c, hipGetLastError());
     run_end_state(c, first_tick, nticks);
     if (tick_ms) {
@@ -5592,7 +5579,7 @@ glint_status glint_batch_run_ticks(glint_batch *b, const double *const *d_traces
     }
     auto enqueue_ticks = [&](uint32_t k) {
         for (; k > 0; k--)
-            for (const FusedGroup &g : groups) enqueue_tick_body(g);
+            for (const FusedGroup &g : groups) enqueue_tick(g);
     };
     // the batch's stream runs after every scenario's pre-run launches, and
     // the scenarios' streams continue after it

@@ -132,7 +132,7 @@ struct Counters {
 };
 
 // Per-tick values, kept in device memory so a tick's launches can be
-// replayed from a graph; advanced on the device by k_advance_tick.
+// replayed from a graph; advanced on the device (advance_tick).
 // One ended meeting kept for the sorted key-value output: the pair, its
 // first and last contact tick and the float box of both objects over the
 // run (low_x, low_y, high_x, high_y).
@@ -177,7 +177,7 @@ struct TickParams {
     uint32_t prev_tick;
     uint32_t trace_index;
     uint32_t has_prev;
-    uint32_t next_tick;         // tick number given by the next k_advance_tick
+    uint32_t next_tick;         // tick number given by the next advance_tick
     uint32_t has_prev_next;
     uint32_t nticks;            // run_ticks: ticks of the run
 };
