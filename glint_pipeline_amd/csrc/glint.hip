@@ -1633,7 +1633,15 @@ __device__ __forceinline__ void scatter_body(const DevState s, const P blk)
     const bool has_prev = s.tp->has_prev != 0;
     // in the previous tick's leaf order, position k held the object now at k
     const bool ordered = s.ctr->sorted_valid != 0;
+    const double *xy = s.tp->xy;
     for (uint32_t k = blk.id() * blockDim.x + threadIdx.x; k < s.n; k += blk.count() * blockDim.x) {
+        // the positions kept for the next tick, copied in the order of the ids
+        // (written from the leaf order, 16 bytes each in a line of its own,
+        // they had taken 0.8 ms of a tick of 20M objects)
+        if (xy_save) {
+            xy_save[2 * (size_t)k] = xy[2 * (size_t)k];
+            xy_save[2 * (size_t)k + 1] = xy[2 * (size_t)k + 1];
+        }
         const uint32_t leaf = s.ord_leaf[k];
         if (leaf == kNone) continue;
         const uint32_t i = s.order[k];
@@ -1651,10 +1659,6 @@ __device__ __forceinline__ void scatter_body(const DevState s, const P blk)
         if (has_prev) {
             px = ordered ? sx_old[k] : xy_prev[2 * (size_t)i];
             py = ordered ? sy_old[k] : xy_prev[2 * (size_t)i + 1];
-        }
-        if (xy_save) {
-            xy_save[2 * (size_t)i] = x;
-            xy_save[2 * (size_t)i + 1] = y;
         }
         if (s.precision == GLINT_PRECISION_FP32_GUARD) {
             Node nd = s.nodes[leaf];
