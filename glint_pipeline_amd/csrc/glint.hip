@@ -30,6 +30,7 @@
 #include "glint_device.h"
 #include "kv_engine.h"
 #include "ctx_view.h"
+#include "order.h"
 
 using namespace glint;
 
@@ -56,6 +57,11 @@ constexpr int kBorderStage = 512;                   // staged border objects per
 enum JoinSum : uint32_t { kSumContacts, kSumBorder, kSumDup, kSumStored, kSumBand, kSumTests, kSumEvals, kJoinSums };
 constexpr uint32_t kJoinParts = 64;
 constexpr uint32_t kJoinPartStride = 16;            // 128 B
+// A tick with at least this many meetings has them sorted on the device for
+// the caller; below, the host sorts them as fast as the sort's launches take
+// (update_meetings with 512 meetings 84 us against 74 by the host, 1024: 89
+// and 93, 2048: 198 and 203, 8192: 241 and 470, 65536: 570 and 3170).
+constexpr uint64_t kOrderMeetings = 2048;
 constexpr uint32_t kHeavyLeaf = 256;                // leaves above this size are joined first
 constexpr uint32_t kSparseMax = 512;                // most objects of a leaf joined by one wave
 // and most objects per reach x reach square of it.  Denser leaves have
@@ -4048,6 +4054,8 @@ struct glint_ctx {
     TableGen tab[2] = {};
     float4 *mbr[2] = {nullptr, nullptr};    // pair boxes of each generation (key-value output)
     KvEngine *kv = nullptr;                 // sorted key-value output (null when off)
+    OrderWork order;                        // buffers that put a tick's meetings in order for the caller
+    uint32_t id_bits = 30;                  // bits of an object id
     double *hist[2] = {nullptr, nullptr};   // positions of the last two ticks (generation parity)
     int cur_gen = 0;            // table generation filled at the current tick
     uint4 *cand[2] = {};        // candidate-list buffers: cand[cur_gen] is written at the current tick
@@ -4662,6 +4670,8 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
     const uint64_t N = cfg->num_objects;
     DevState &s = c->s;
     s.n = (uint32_t)N;
+    c->id_bits = 1;
+    while ((1ull << c->id_bits) < N) c->id_bits++;
     s.cap = cfg->grid_capacity;
     s.min_meet = cfg->min_meet_time;
     s.complete = cfg->candidate_mode;
@@ -4897,6 +4907,7 @@ glint_status glint_destroy(glint_ctx *c)
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->stamps) (void)hipFree(c->stamps);
     kv_destroy(c->kv);
+    order_free(c->order);
     if (c->h_ctr) (void)hipHostFree(c->h_ctr);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -5062,7 +5073,10 @@ glint_status glint_evaluate(glint_ctx *c, glint_meeting *out, uint64_t cap, uint
         return GLINT_ERR_OUTPUT_CAPACITY;
     }
     if (n) {
+        const bool ordered = n >= kOrderMeetings && order_meetings(c->order, c->stream, c->s.meet, n, c->id_bits);
+        if (ordered) HIP_TRY(c, hipStreamSynchronize(c->stream));
         HIP_TRY(c, hipMemcpy(out, c->s.meet, n * sizeof(glint_meeting), hipMemcpyDeviceToHost));
+        if (ordered) return GLINT_OK;
         std::sort(out, out + n, [](const glint_meeting &a, const glint_meeting &b) {
             if (a.pid_a != b.pid_a) return a.pid_a < b.pid_a;
             if (a.pid_b != b.pid_b) return a.pid_b < b.pid_b;
