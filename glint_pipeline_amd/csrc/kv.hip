@@ -98,18 +98,59 @@ __global__ __launch_bounds__(kB) void k_iota(uint32_t *p, uint64_t n)
         p[i] = (uint32_t)i;
 }
 
-// dst64[i] = src64[perm[i]], dst32[i] = src32[perm[i]].
-__global__ __launch_bounds__(kB) void k_permute(const uint32_t *perm, const uint64_t *src64, uint64_t *dst64,
-                                                const uint32_t *src32, uint32_t *dst32, uint64_t n)
+// The bits that differ across a set of 128-bit keys, as runs from the most
+// significant down: run k is `width` bits from bit `shift` of the high
+// (word 1) or low word.
+constexpr uint32_t kMaxRuns = 16;
+struct KeyRuns {
+    uint32_t n;
+    uint8_t word[kMaxRuns], shift[kMaxRuns], width[kMaxRuns];
+};
+
+// Every row's differing bits side by side in one 64-bit key (the order of the
+// rows, since the other bits are equal), and its index.
+__global__ __launch_bounds__(kB) void k_squeeze(const uint64_t *hi, const uint64_t *lo, KeyRuns r, uint64_t *keys,
+                                                uint32_t *idx, uint64_t n)
 {
     for (uint64_t i = blockIdx.x * (uint64_t)kB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kB) {
-        const uint32_t j = perm[i];
-        dst64[i] = src64[j];
-        dst32[i] = src32[j];
+        const uint64_t h = hi[i], l = lo[i];
+        uint64_t k = 0;
+        for (uint32_t q = 0; q < r.n; q++) {
+            const uint64_t x = (r.word[q] ? h : l) >> r.shift[q];
+            const uint64_t m = r.width[q] < 64 ? (1ull << r.width[q]) - 1 : ~0ull;
+            k = r.width[q] < 64 ? (k << r.width[q]) | (x & m) : x;
+        }
+        keys[i] = k;
+        idx[i] = (uint32_t)i;
     }
 }
 
+// Rows in the order perm (null: as they are).
+__global__ __launch_bounds__(kB) void k_rows(const uint32_t *perm, SortView in, SortView out, uint64_t n)
+{
+    for (uint64_t i = blockIdx.x * (uint64_t)kB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kB) {
+        const uint64_t j = perm ? perm[i] : i;
+        out.hi[i] = in.hi[j];
+        out.lo[i] = in.lo[j];
+        out.val[i] = in.val[j];
+    }
+}
+
+// Keys as the caller gets them, the low word first; file ids narrowed.
+__global__ __launch_bounds__(kB) void k_interleave(const uint64_t *hi, const uint64_t *lo, uint64_t n, ulonglong2 *out)
+{
+    for (uint64_t i = blockIdx.x * (uint64_t)kB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kB)
+        out[i] = make_ulonglong2(lo[i], hi[i]);
+}
+
+__global__ __launch_bounds__(kB) void k_narrow_sids(const uint32_t *sids, uint32_t n, uint16_t *out)
+{
+    for (uint32_t i = blockIdx.x * kB + threadIdx.x; i < n; i += gridDim.x * kB) out[i] = (uint16_t)sids[i];
+}
+
 // AND and OR of all keys: the bits that differ decide which digits to sort.
+// One atomic per word and workgroup: those of 4096 waves on one line had run
+// one after another (157 us whatever the keys).
 __global__ __launch_bounds__(kB) void k_andor(const uint64_t *hi, const uint64_t *lo, uint64_t n, KvCtr *ctr)
 {
     uint64_t ah = ~0ull, al = ~0ull, oh = 0, ol = 0;
@@ -126,12 +167,26 @@ __global__ __launch_bounds__(kB) void k_andor(const uint64_t *hi, const uint64_t
         oh |= __shfl_xor(oh, d);
         ol |= __shfl_xor(ol, d);
     }
+    __shared__ uint64_t w[4][kB / 64];
     if (lane() == 0) {
-        atomicAnd(&ctr->and_hi, (unsigned long long)ah);
-        atomicAnd(&ctr->and_lo, (unsigned long long)al);
-        atomicOr(&ctr->or_hi, (unsigned long long)oh);
-        atomicOr(&ctr->or_lo, (unsigned long long)ol);
+        const uint32_t k = threadIdx.x / 64;
+        w[0][k] = ah;
+        w[1][k] = al;
+        w[2][k] = oh;
+        w[3][k] = ol;
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (uint32_t k = 1; k < kB / 64; k++) {
+        ah &= w[0][k];
+        al &= w[1][k];
+        oh |= w[2][k];
+        ol |= w[3][k];
+    }
+    atomicAnd(&ctr->and_hi, (unsigned long long)ah);
+    atomicAnd(&ctr->and_lo, (unsigned long long)al);
+    atomicOr(&ctr->or_hi, (unsigned long long)oh);
+    atomicOr(&ctr->or_lo, (unsigned long long)ol);
 }
 
 __global__ void k_ctr_reset_masks(KvCtr *c)
@@ -229,10 +284,16 @@ __global__ __launch_bounds__(kB) void k_objects(uint32_t n, const uint32_t *cnt,
         present += __shfl_xor(present, d);
         cut += __shfl_xor(cut, d);
     }
+    __shared__ uint32_t sum[2];
+    if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+    __syncthreads();
     if (lane() == 0) {
-        if (present) atomicAdd(&ctr->sid_count, present);
-        if (cut) atomicAdd(&ctr->ovs_area, cut);
+        if (present) atomicAdd(&sum[0], present);
+        if (cut) atomicAdd(&sum[1], cut);
     }
+    __syncthreads();
+    if (threadIdx.x == 0 && sum[0]) atomicAdd(&ctr->sid_count, sum[0]);   // (one atomic per workgroup: see k_andor)
+    if (threadIdx.x == 0 && sum[1]) atomicAdd(&ctr->ovs_area, sum[1]);
 }
 
 // Keys of sid-1 objects to the tail, the rest to the head (geometry.cu:1776-1797).
@@ -537,11 +598,17 @@ __global__ __launch_bounds__(kB) void k_pack(const glint_ctf *ctfs, uint32_t nct
 
 // get_o_limit start times (geometry.cu:929-979) and cuda_write_o_bitmap
 // (geometry.cu:895-913) over the root box, cells clipped as in
-// step_merge.cpp:57-58.
+// step_merge.cpp:57-58.  A workgroup gathers its bits in LDS: the keys of a
+// crowd share a few words of the bitmap, and an atomic in memory per key had
+// taken 0.92 ms for 261k keys.
 __global__ __launch_bounds__(kB) void k_oversize(const uint64_t *lo, const float4 *boxes, uint64_t b0, uint64_t b1,
                                                  double mlx, double mly, double mhx, double mhy,
                                                  uint32_t end_time_min, uint32_t *obitmap, KvCtr *ctr)
 {
+    __shared__ uint32_t bm[kBitmapBytes / 4], st[2];
+    for (uint32_t k = threadIdx.x; k < kBitmapBytes / 4; k += kB) bm[k] = 0;
+    if (threadIdx.x < 2) st[threadIdx.x] = threadIdx.x ? 0u : 1u << 30;
+    __syncthreads();
     uint32_t smin = 1u << 30, smax = 0;
     for (uint64_t i = b0 + blockIdx.x * (uint64_t)kB + threadIdx.x; i < b1; i += (uint64_t)gridDim.x * kB) {
         const uint32_t dur = (uint32_t)(lo[i] >> 32);
@@ -556,7 +623,8 @@ __global__ __launch_bounds__(kB) void k_oversize(const uint64_t *lo, const float
         for (uint32_t x = l0; x <= h0 && x < kBitmapEdge; x++)
             for (uint32_t y = l1; y <= h1 && y < kBitmapEdge; y++) {
                 const uint32_t pos = x + y * kBitmapEdge;
-                atomicOr(&obitmap[pos >> 5], 1u << (pos & 31));
+                const uint32_t bit = 1u << (pos & 31);
+                if (!(bm[pos >> 5] & bit)) atomicOr(&bm[pos >> 5], bit);
             }
     }
     for (int d = 32; d >= 1; d >>= 1) {
@@ -564,8 +632,15 @@ __global__ __launch_bounds__(kB) void k_oversize(const uint64_t *lo, const float
         smax = max(smax, (uint32_t)__shfl_xor(smax, d));
     }
     if (lane() == 0) {
-        atomicMin(&ctr->osmin, smin);
-        atomicMax(&ctr->osmax, smax);
+        atomicMin(&st[0], smin);
+        atomicMax(&st[1], smax);
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < kBitmapBytes / 4; k += kB)
+        if (bm[k]) atomicOr(&obitmap[k], bm[k]);
+    if (threadIdx.x == 0) {
+        atomicMin(&ctr->osmin, st[0]);
+        atomicMax(&ctr->osmax, st[1]);
     }
 }
 
@@ -683,19 +758,22 @@ glint_status read_ctr(KvEngine *e, std::string &err)
 // the high word (empty ranges: lo >= hi).
 struct VaryingBits {
     uint32_t lo_begin, lo_end, hi_begin, hi_end;
+    uint64_t lo, hi;   // the bits themselves
 };
 
 glint_status varying_bits(KvEngine *e, const SortView &v, uint64_t n, bool wide, VaryingBits &vb,
                           std::string &err)
 {
-    vb = VaryingBits{0, 0, 0, 0};
+    vb = VaryingBits{};
     if (n < 2) return GLINT_OK;
     k_ctr_reset_masks<<<1, 1, 0, e->st>>>(e->ctr);
-    k_andor<<<grid_of(n, 1024), kB, 0, e->st>>>(wide ? v.hi : nullptr, v.lo, n, e->ctr);
+    k_andor<<<grid_of(n, 512), kB, 0, e->st>>>(wide ? v.hi : nullptr, v.lo, n, e->ctr);
     KV_TRY(hipGetLastError());
     glint_status s = read_ctr(e, err);
     if (s) return s;
     const uint64_t dh = wide ? e->h_ctr->or_hi ^ e->h_ctr->and_hi : 0, dl = e->h_ctr->or_lo ^ e->h_ctr->and_lo;
+    vb.lo = dl;
+    vb.hi = dh;
     if (dl) vb.lo_begin = (uint32_t)__builtin_ctzll(dl), vb.lo_end = 64 - (uint32_t)__builtin_clzll(dl);
     if (dh) vb.hi_begin = (uint32_t)__builtin_ctzll(dh), vb.hi_end = 64 - (uint32_t)__builtin_clzll(dh);
     return GLINT_OK;
@@ -720,48 +798,84 @@ glint_status sort_pairs(KvEngine *e, uint64_t *k0, uint64_t *k1, uint32_t *v0, u
     return GLINT_OK;
 }
 
-// Stable sort of n items of `a` by their keys (the high word, if wide, then
-// the low word), `b` as scratch; the result is left in `a`.  A wide key is
-// sorted by its low word carrying the row index, the rows permuted, then by
-// its high word carrying the row index again, and the rows permuted; only
-// the bits that differ across the keys are sorted.
-glint_status radix_sort(KvEngine *e, SortView a, SortView b, uint64_t n, bool wide, std::string &err)
+// Stable sort of the n (key, value) pairs of `a` by key, `b` as scratch; the
+// result is left in `a`.
+glint_status sort_objects(KvEngine *e, SortView a, SortView b, uint64_t n, std::string &err)
 {
     VaryingBits vb;
-    glint_status s = varying_bits(e, a, n, wide, vb, err);
+    glint_status s = varying_bits(e, a, n, false, vb, err);
+    if (s) return s;
+    if (vb.lo_begin >= vb.lo_end) return GLINT_OK;
+    bool scratch = false;
+    s = sort_pairs(e, a.lo, b.lo, a.val, b.val, n, vb.lo_begin, vb.lo_end, scratch, err);
+    if (s) return s;
+    if (scratch) {
+        KV_TRY(hipMemcpyAsync(a.lo, b.lo, n * 8, hipMemcpyDeviceToDevice, e->st));
+        KV_TRY(hipMemcpyAsync(a.val, b.val, n * 4, hipMemcpyDeviceToDevice, e->st));
+    }
+    return GLINT_OK;
+}
+
+// The runs of bits that differ, from the top; false if they do not fit a
+// 64-bit key.
+bool key_runs(const VaryingBits &vb, KeyRuns &r)
+{
+    if (__builtin_popcountll(vb.hi) + __builtin_popcountll(vb.lo) > 64) return false;
+    r = KeyRuns{};
+    for (int word = 1; word >= 0; word--) {
+        uint64_t m = word ? vb.hi : vb.lo;
+        while (m) {
+            if (r.n == kMaxRuns) return false;
+            const uint32_t top = 64 - (uint32_t)__builtin_clzll(m);   // one past the highest bit left
+            uint32_t low = top;
+            while (low > 0 && (m >> (low - 1)) & 1ull) low--;
+            r.word[r.n] = (uint8_t)word;
+            r.shift[r.n] = (uint8_t)low;
+            r.width[r.n] = (uint8_t)(top - low);
+            r.n++;
+            m = low ? m & ((1ull << low) - 1) : 0;
+        }
+    }
+    return true;
+}
+
+// Stable sort of the n rows (hi, lo, value) of `in` by their 128-bit keys into
+// `out`.  Keys mostly differ in few bits (about 55 of 128: ids, durations
+// and ends use the low bits of their fields), which are squeezed into one
+// 64-bit key, sorted with the row's index, and the rows follow once.  Keys
+// that differ in more bits are sorted by their low word carrying the row
+// index, then stably by their high word, the rows following each time.
+glint_status sort_rows(KvEngine *e, SortView in, SortView out, uint64_t n, std::string &err)
+{
+    if (n == 0) return GLINT_OK;
+    VaryingBits vb;
+    glint_status s = varying_bits(e, in, n, true, vb, err);
     if (s) return s;
     const uint32_t g = grid_of(n);
     bool scratch = false;
-    if (!wide) {
-        if (vb.lo_begin >= vb.lo_end) return GLINT_OK;
-        s = sort_pairs(e, a.lo, b.lo, a.val, b.val, n, vb.lo_begin, vb.lo_end, scratch, err);
+    KeyRuns r;
+    if (!vb.hi && !vb.lo) {
+        k_rows<<<g, kB, 0, e->st>>>(nullptr, in, out, n);
+    } else if (key_runs(vb, r)) {
+        const uint32_t bits = (uint32_t)(__builtin_popcountll(vb.hi) + __builtin_popcountll(vb.lo));
+        k_squeeze<<<g, kB, 0, e->st>>>(in.hi, in.lo, r, out.lo, e->idx0, n);
+        s = sort_pairs(e, out.lo, out.hi, e->idx0, e->idx1, n, 0, bits, scratch, err);
         if (s) return s;
-        if (scratch) {
-            KV_TRY(hipMemcpyAsync(a.lo, b.lo, n * 8, hipMemcpyDeviceToDevice, e->st));
-            KV_TRY(hipMemcpyAsync(a.val, b.val, n * 4, hipMemcpyDeviceToDevice, e->st));
+        k_rows<<<g, kB, 0, e->st>>>(scratch ? e->idx1 : e->idx0, in, out, n);
+    } else {
+        SortView from = in, to = out;
+        for (int word = 0; word < 2; word++) {
+            const uint32_t b0 = word ? vb.hi_begin : vb.lo_begin, b1 = word ? vb.hi_end : vb.lo_end;
+            if (b0 >= b1) continue;
+            // the words to sort go through `to`, which the rows then follow into
+            KV_TRY(hipMemcpyAsync(to.lo, word ? from.hi : from.lo, n * 8, hipMemcpyDeviceToDevice, e->st));
+            k_iota<<<g, kB, 0, e->st>>>(e->idx0, n);
+            s = sort_pairs(e, to.lo, to.hi, e->idx0, e->idx1, n, b0, b1, scratch, err);
+            if (s) return s;
+            k_rows<<<g, kB, 0, e->st>>>(scratch ? e->idx1 : e->idx0, from, to, n);
+            std::swap(from, to);
         }
-        return GLINT_OK;
-    }
-    // rows (hi, lo, val) live in a; b and the two index buffers are scratch
-    if (vb.lo_begin < vb.lo_end) {
-        k_iota<<<g, kB, 0, e->st>>>(e->idx0, n);
-        s = sort_pairs(e, a.lo, b.lo, e->idx0, e->idx1, n, vb.lo_begin, vb.lo_end, scratch, err);
-        if (s) return s;
-        const uint32_t *perm = scratch ? e->idx1 : e->idx0;
-        if (scratch) KV_TRY(hipMemcpyAsync(a.lo, b.lo, n * 8, hipMemcpyDeviceToDevice, e->st));
-        k_permute<<<g, kB, 0, e->st>>>(perm, a.hi, b.hi, a.val, b.val, n);
-        KV_TRY(hipMemcpyAsync(a.hi, b.hi, n * 8, hipMemcpyDeviceToDevice, e->st));
-        KV_TRY(hipMemcpyAsync(a.val, b.val, n * 4, hipMemcpyDeviceToDevice, e->st));
-    }
-    if (vb.hi_begin < vb.hi_end) {
-        k_iota<<<g, kB, 0, e->st>>>(e->idx0, n);
-        s = sort_pairs(e, a.hi, b.hi, e->idx0, e->idx1, n, vb.hi_begin, vb.hi_end, scratch, err);
-        if (s) return s;
-        const uint32_t *perm = scratch ? e->idx1 : e->idx0;
-        if (scratch) KV_TRY(hipMemcpyAsync(a.hi, b.hi, n * 8, hipMemcpyDeviceToDevice, e->st));
-        k_permute<<<g, kB, 0, e->st>>>(perm, a.lo, b.lo, a.val, b.val, n);
-        KV_TRY(hipMemcpyAsync(a.lo, b.lo, n * 8, hipMemcpyDeviceToDevice, e->st));
-        KV_TRY(hipMemcpyAsync(a.val, b.val, n * 4, hipMemcpyDeviceToDevice, e->st));
+        if (from.lo != out.lo) k_rows<<<g, kB, 0, e->st>>>(nullptr, from, out, n);
     }
     KV_TRY(hipGetLastError());
     return GLINT_OK;
@@ -865,32 +979,32 @@ glint_status kv_flush(KvEngine *e, uint64_t nlog, uint32_t cur_time, glint_kv_su
     const uint32_t ovs = e->h_ctr->ovs_meet + e->h_ctr->ovs_area;
 
     // oversize buffer: sorted keys
-    s = radix_sort(e, offset(e->b, nk), offset(e->a, nk), no, true, err);
+    s = sort_rows(e, offset(e->b, nk), offset(e->a, nk), no, err);
     if (s) return s;
 
     // STR (geometry.cu:1832-1895)
-    s = radix_sort(e, e->oa, e->ob, N, false, err);
+    s = sort_objects(e, e->oa, e->ob, N, err);
     if (s) return s;
     const uint32_t z = (N - sid_count) + ovs;
     const uint32_t xcap = (sid_count - ovs) / split + 1;
     const uint32_t part = xcap / split + 1;
     if (z < N) {
         k_narrow<<<gN, kB, 0, st>>>(e->oa.lo, N, z, xcap, split);
-        s = radix_sort(e, e->oa, e->ob, N, false, err);
+        s = sort_objects(e, e->oa, e->ob, N, err);
         if (s) return s;
         k_make_sid<<<gN, kB, 0, st>>>(e->oa.val, N, z, xcap, part, split, e->sids);
     }
 
     // kept keys: sid written, sorted; boxes follow their keys
     if (nk) k_write_sid<<<grid_of(nk), kB, 0, st>>>(e->b.hi, nk, e->sids);
-    s = radix_sort(e, e->b, e->a, nk, true, err);
+    s = sort_rows(e, e->b, e->a, nk, err);   // (the sorted rows of both sides are in a)
     if (s) return s;
-    if (nkeys) k_gather_boxes<<<gK, kB, 0, st>>>(e->b.val, e->box_in, e->box_out, nkeys);
+    if (nkeys) k_gather_boxes<<<gK, kB, 0, st>>>(e->a.val, e->box_in, e->box_out, nkeys);
 
     // files: capacities, limits; widths on the host
     k_fill_u32<<<grid_of(C), kB, 0, st>>>(e->cap, C, 0);
     if (z < N) k_capacity<<<grid_of(N - z, 1024), kB, 0, st>>>(e->oa.val, N, z, e->sids, e->cnt, C, e->cap);
-    k_limits<<<C, kB, 0, st>>>(e->cap, C, e->b.hi, e->b.lo, e->box_out, nk, e->end_time_min, cur_time, e->ctfs);
+    k_limits<<<C, kB, 0, st>>>(e->cap, C, e->a.hi, e->a.lo, e->box_out, nk, e->end_time_min, cur_time, e->ctfs);
     KV_TRY(hipGetLastError());
     e->h_ctfs.assign(C, glint_ctf{});
     KV_TRY(hipMemcpyAsync(e->h_ctfs.data(), e->ctfs, C * sizeof(glint_ctf), hipMemcpyDeviceToHost, st));
@@ -920,12 +1034,12 @@ glint_status kv_flush(KvEngine *e, uint64_t nlog, uint32_t cur_time, glint_kv_su
         const uint32_t slices = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(64, nk / ((uint64_t)C * 4096) + 1));
         k_bitmaps<<<dim3(C, slices), kB, 0, st>>>(e->ctfs, e->box_out, nk, e->bitmaps);
     }
-    if (nk) k_pack<<<grid_of(nk), kB, 0, st>>>(e->ctfs, C, e->b.hi, e->b.lo, e->box_out, nk, e->packed);
+    if (nk) k_pack<<<grid_of(nk), kB, 0, st>>>(e->ctfs, C, e->a.hi, e->a.lo, e->box_out, nk, e->packed);
 
     // oversize buffer: start times and map bitmap
     k_fill_u32<<<8, kB, 0, st>>>(e->obitmap, kBitmapBytes / 4, 0);
     if (no)
-        k_oversize<<<grid_of(no, 1024), kB, 0, st>>>(e->b.lo, e->box_out, nk, nk + no, e->p.map[0], e->p.map[1],
+        k_oversize<<<grid_of(no, 512), kB, 0, st>>>(e->a.lo, e->box_out, nk, nk + no, e->p.map[0], e->p.map[1],
                                                      e->p.map[2], e->p.map[3], e->end_time_min, e->obitmap, e->ctr);
     KV_TRY(hipGetLastError());
     s = read_ctr(e, err);
@@ -983,15 +1097,13 @@ glint_status kv_copy(KvEngine *e, uint32_t part, void *dst, uint64_t bytes, std:
     if (!bytes) return GLINT_OK;
     const uint64_t nk = e->sum.kept_keys, no = e->sum.oversize_keys;
     KV_TRY(hipStreamSynchronize(e->st));
+    // keys and file ids are put in their form on the device, in the boxes'
+    // input (not needed after the flush)
     auto keys = [&](uint64_t first, uint64_t n) -> glint_status {
-        std::vector<uint64_t> h(n), l(n);
-        KV_TRY(hipMemcpy(h.data(), e->b.hi + first, n * 8, hipMemcpyDeviceToHost));
-        KV_TRY(hipMemcpy(l.data(), e->b.lo + first, n * 8, hipMemcpyDeviceToHost));
-        uint64_t *o = (uint64_t *)dst;
-        for (uint64_t i = 0; i < n; i++) {
-            o[2 * i] = l[i];
-            o[2 * i + 1] = h[i];
-        }
+        k_interleave<<<grid_of(n), kB, 0, e->st>>>(e->a.hi + first, e->a.lo + first, n, (ulonglong2 *)e->box_in);
+        KV_TRY(hipGetLastError());
+        KV_TRY(hipStreamSynchronize(e->st));
+        KV_TRY(hipMemcpy(dst, e->box_in, n * 16, hipMemcpyDeviceToHost));
         return GLINT_OK;
     };
     switch (part) {
@@ -1002,10 +1114,11 @@ glint_status kv_copy(KvEngine *e, uint32_t part, void *dst, uint64_t bytes, std:
         KV_TRY(hipMemcpy(dst, e->box_out + nk, bytes, hipMemcpyDeviceToHost));
         return GLINT_OK;
     case GLINT_KV_SIDS: {
-        std::vector<uint32_t> v(e->p.num_objects);
-        KV_TRY(hipMemcpy(v.data(), e->sids, v.size() * 4, hipMemcpyDeviceToHost));
-        uint16_t *o = (uint16_t *)dst;
-        for (size_t i = 0; i < v.size(); i++) o[i] = (uint16_t)v[i];
+        uint16_t *narrow = reinterpret_cast<uint16_t *>(e->ob.lo);   // (8 bytes an object; scratch of the flush)
+        k_narrow_sids<<<grid_of(e->p.num_objects), kB, 0, e->st>>>(e->sids, e->p.num_objects, narrow);
+        KV_TRY(hipGetLastError());
+        KV_TRY(hipStreamSynchronize(e->st));
+        KV_TRY(hipMemcpy(dst, narrow, bytes, hipMemcpyDeviceToHost));
         return GLINT_OK;
     }
     case GLINT_KV_CTFS: std::memcpy(dst, e->h_ctfs.data(), bytes); return GLINT_OK;
