@@ -149,8 +149,7 @@ STAGE_OF_KERNEL = {
     "k_begin_tick": "filter", "k_assign": "filter", "k_scan_objects": "filter", "k_place": "filter",
     "k_scan_units": "filter", "k_unit_scatter": "filter", "k_grid_cells": "filter", "k_grid_pyramid": "filter",
     "k_grid_top": "filter", "k_grid_fine_zero": "filter", "k_grid_fine": "filter", "k_grid_level": "filter",
-    "k_join": "reachability", "k_bucket_count": "reachability", "k_scan_reduce": "reachability",
-    "k_scan_top": "reachability", "k_scan_write": "reachability", "k_bucket_scatter": "reachability",
+    "k_join": "reachability", "k_bucket_count": "reachability", "k_bucket_scatter": "reachability",
     "k_bucket_fine": "reachability", "k_table": "update_meetings", "k_pos32": "update_meetings",
     "k_collect": "update_schema", "k_schema": "update_schema",
 }

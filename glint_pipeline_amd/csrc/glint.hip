@@ -51,6 +51,7 @@ constexpr int kBucketThreads = 1024;                // workgroup of the two buck
 constexpr int kBucketTile = 16384;                  // contacts per LDS tile of the coarse pass (128 KB)
 constexpr int kFineTile = 12288;                    // contacts per LDS tile of the fine pass (96 KB)
 constexpr uint32_t kMaxCoarse = 1024;               // coarse bins of pass 1
+constexpr uint32_t kBinStride = 32;                 // words between their totals (a line each)
 constexpr uint32_t kMaxFine = 2048;                 // fine bins of pass 2
 constexpr int kBorderStage = 512;                   // staged border objects per wave (assign)
 // Counts of the join, kept in kJoinParts lines until k_bucket_count adds them up.
@@ -418,6 +419,7 @@ __device__ __forceinline__ void stamp_end(TickParams *tp)
 __device__ __forceinline__ void reset_tick_body(const DevState &s)
 {
     for (uint32_t k = threadIdx.x; k < kJoinParts * kJoinPartStride; k += blockDim.x) s.jpart[k] = 0;
+    for (uint32_t k = threadIdx.x; k < s.coarse_max; k += blockDim.x) s.bins[k * kBinStride] = 0;
     if (threadIdx.x != 0) return;
     Counters *c = s.ctr;
     c->n_units = 0;
@@ -1420,61 +1422,6 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *t
     __syncthreads();
     *total = all;
     return before + inc - v;
-}
-
-// Three-kernel exclusive scan of the region bins of the contact grouping
-// (k_scan_reduce, k_scan_top, k_scan_write).
-template <class P>
-__device__ __forceinline__ void scan_reduce_body(const uint32_t *in, uint32_t n, uint32_t *block_sums, const P blk)
-{
-    uint32_t base = blk.id() * kScanTile + threadIdx.x * kScanItems;
-    uint32_t v = 0;
-    for (int k = 0; k < kScanItems; k++)
-        if (base + k < n) v += in[base + k];
-    uint32_t total;
-    block_exclusive_scan(v, &total);
-    if (threadIdx.x == 0) block_sums[blk.id()] = total;
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan_reduce(const uint32_t *in, uint32_t n, uint32_t *block_sums)
-{
-    scan_reduce_body(in, n, block_sums, this_blk());
-}
-
-__host__ __device__ inline uint32_t bins_length(const DevState &s) { return (s.coarse_max + 1) * s.bucket_blocks; }
-
-__host__ __device__ inline uint32_t scan_blocks_for(uint32_t n) { return (n + kScanTile - 1) / kScanTile; }
-
-__global__ __launch_bounds__(kBlock) void kf_scan_reduce(const Many m)
-{
-    const Member w = member_of(m);
-    const DevState &s = m.ss[w.i];
-    scan_reduce_body(s.bcount, bins_length(s), s.block_sums, w.blk);
-}
-
-__device__ __forceinline__ void scan_top_body(uint32_t *block_sums, uint32_t nblocks)
-{
-    uint32_t carry = 0;
-    for (uint32_t b0 = 0; b0 < nblocks; b0 += kBlock) {
-        uint32_t b = b0 + threadIdx.x;
-        uint32_t v = b < nblocks ? block_sums[b] : 0;
-        uint32_t total;
-        uint32_t ex = block_exclusive_scan(v, &total);
-        if (b < nblocks) block_sums[b] = carry + ex;
-        carry += total;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan_top(uint32_t *block_sums, uint32_t nblocks)
-{
-    scan_top_body(block_sums, nblocks);
-}
-
-__global__ __launch_bounds__(kBlock) void kf_scan_top(const Many m)
-{
-    const Member w = member_of(m);
-    const DevState &s = m.ss[w.i];
-    scan_top_body(s.block_sums, scan_blocks_for(bins_length(s)));
 }
 
 // Object offsets of every leaf and the leaf statistics.  The workgroups take
@@ -3239,17 +3186,28 @@ __global__ __launch_bounds__(kBlock, 4) void kf_join(const Many m)   // (4 waves
 
 // ------------------------------------------------------------ bucketing
 //
-// Two passes group the contact list by region.  Pass 1 (k_bucket_count, a
-// scan, k_bucket_scatter) splits it by the high bits of the region index into
-// at most 1024 coarse bins, sentinels going to one extra bin that is never
-// written out; each block sorts 8192-entry tiles in LDS so its writes form
-// runs.  Pass 2 (k_bucket_fine) splits every coarse bin by the low bits with
-// one workgroup per bin and records the first contact of every region.
+// Two passes group the contact list by region.  Pass 1 (k_bucket_count,
+// k_bucket_scatter) splits it by the high bits of the region index into
+// at most 1024 coarse bins; each block sorts 16384-entry tiles in LDS so its
+// writes form runs.  Pass 2 (k_bucket_fine) splits every coarse bin by the low
+// bits with one workgroup per bin and records the first contact of every region.
+// The counting pass adds every block's counts to the bins' totals, a line
+// each, and keeps the places that gives the block in its bins: the passes
+// after it add up the totals themselves (three launches had scanned a table
+// of blocks x bins).  A list that fits one tile of pass 2, and a table of no
+// more regions than that pass has bins, skips pass 1 (one_tile): a sparse
+// tick waits for launches, not for memory.
 
 __device__ __forceinline__ uint32_t coarse_bin(const TableShape &sh, unsigned long long tagged)
 {
     if (tagged == kEmptyKey) return sh.coarse;
     return region_of(tagged & kKeyBits, sh.bits) >> sh.lo_bits;
+}
+
+// Whether the whole list is grouped by one workgroup of pass 2.
+__device__ __forceinline__ bool one_tile(unsigned long long n, const TableShape &sh)
+{
+    return n <= kFineTile && (1u << sh.bits) <= kMaxFine;
 }
 
 template <class P>
@@ -3285,65 +3243,48 @@ __device__ __forceinline__ void bucket_count_body(const DevState s, const P blk)
         }
     }
     const TableShape sh = table_shape(s, stored);
-    for (uint32_t k = threadIdx.x; k <= sh.coarse; k += kBlock) hist[k] = 0;
+    if (one_tile(n, sh)) return;
+    for (uint32_t k = threadIdx.x; k <= sh.coarse; k += kBucketThreads) hist[k] = 0;
     __syncthreads();
     unsigned long long b0, b1;
     block_range(blk, n, b0, b1);
     const unsigned long long *in = contact_out(s);
     // four independent loads in flight per thread
     constexpr int kU = 4;
-    for (unsigned long long i0 = b0 + threadIdx.x; i0 < b1; i0 += kU * kBlock) {
+    for (unsigned long long i0 = b0 + threadIdx.x; i0 < b1; i0 += kU * kBucketThreads) {
         unsigned long long key[kU];
 #pragma unroll
-        for (int q = 0; q < kU; q++) key[q] = i0 + q * kBlock < b1 ? in[i0 + q * kBlock] : 0ull;
+        for (int q = 0; q < kU; q++) key[q] = i0 + q * kBucketThreads < b1 ? in[i0 + q * kBucketThreads] : kEmptyKey;
 #pragma unroll
-        for (int q = 0; q < kU; q++)
-            if (i0 + q * kBlock < b1) atomicAdd(&hist[coarse_bin(sh, key[q])], 1u);
+        for (int q = 0; q < kU; q++)   // (the lists' unused slots are not counted: they would all count in one bin)
+            if (key[q] != kEmptyKey) atomicAdd(&hist[coarse_bin(sh, key[q])], 1u);
     }
     __syncthreads();
-    // bins past this tick's (the empty-slot bin is sh.coarse) count nothing
-    for (uint32_t k = threadIdx.x; k <= s.coarse_max; k += kBlock)
-        s.bcount[(size_t)k * blk.count() + blk.id()] = k <= sh.coarse ? hist[k] : 0u;
+    for (uint32_t k = threadIdx.x; k < sh.coarse; k += kBucketThreads)
+        if (hist[k]) s.boff[(size_t)k * blk.count() + blk.id()] = atomicAdd(&s.bins[k * kBinStride], hist[k]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_bucket_count(DevState s) { bucket_count_body(s, this_blk()); }
-__global__ __launch_bounds__(kBlock) void kf_bucket_count(const Many m)
+__global__ __launch_bounds__(kBucketThreads) void k_bucket_count(DevState s) { bucket_count_body(s, this_blk()); }
+__global__ __launch_bounds__(kBucketThreads) void kf_bucket_count(const Many m)
 {
     const Member w = member_of(m);
     bucket_count_body(m.ss[w.i], w.blk);
 }
 
-// Exclusive offsets of a scanned counter array (third kernel of the scan).
-template <class P>
-__device__ __forceinline__ void scan_write_body(const uint32_t *in, uint32_t n, const uint32_t *block_sums,
-                                                uint32_t *out, const P blk)
+// First contact of every coarse bin, and the count at the end, from the bins'
+// totals; kBucketThreads threads, wsum one word per wave.
+__device__ __forceinline__ void bin_starts(const DevState &s, const TableShape &sh, uint32_t *start, uint32_t *wsum)
 {
-    uint32_t base = blk.id() * kScanTile + threadIdx.x * kScanItems;
-    uint32_t c[kScanItems];
-    uint32_t v = 0;
-    for (int k = 0; k < kScanItems; k++) {
-        c[k] = base + k < n ? in[base + k] : 0;
-        v += c[k];
-    }
-    uint32_t total;
-    uint32_t ex = block_exclusive_scan(v, &total) + block_sums[blk.id()];
-    for (int k = 0; k < kScanItems; k++) {
-        if (base + k < n) out[base + k] = ex;
-        ex += c[k];
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan_write(const uint32_t *in, uint32_t n, const uint32_t *block_sums,
-                                                       uint32_t *out)
-{
-    scan_write_body(in, n, block_sums, out, this_blk());
-}
-
-__global__ __launch_bounds__(kBlock) void kf_scan_write_bins(const Many m)
-{
-    const Member w = member_of(m);
-    const DevState &s = m.ss[w.i];
-    scan_write_body(s.bcount, bins_length(s), s.block_sums, s.boff, w.blk);
+    static_assert(kMaxCoarse <= kBucketThreads, "one bin per thread");
+    const uint32_t v = threadIdx.x < sh.coarse ? s.bins[threadIdx.x * kBinStride] : 0u;
+    const uint32_t inc = wave_inclusive_scan(v);
+    if (lane_id() == 63) wsum[threadIdx.x / 64] = inc;
+    __syncthreads();
+    uint32_t ex = inc - v;
+    for (uint32_t w = 0; w < threadIdx.x / 64; w++) ex += wsum[w];
+    if (threadIdx.x < sh.coarse) start[threadIdx.x] = ex;
+    if (threadIdx.x == sh.coarse - 1) start[sh.coarse] = ex + v;
+    __syncthreads();
 }
 
 template <class P>
@@ -3354,12 +3295,17 @@ __device__ __forceinline__ void bucket_scatter_body(const DevState s, const P bl
     __shared__ uint32_t wsum[kBucketThreads / 64];
     const unsigned long long n = min(s.ctr->n_clist, s.clist_cap);
     const TableShape sh = table_shape(s);
+    if (one_tile(n, sh)) return;
     const uint32_t nb = sh.coarse + 1;
     const unsigned long long *in = contact_out(s);
     unsigned long long *out = s.clist2;
     unsigned long long b0, b1;
     block_range(blk, n, b0, b1);
-    for (uint32_t k = threadIdx.x; k < nb; k += kBucketThreads) running[k] = s.boff[(size_t)k * blk.count() + blk.id()];
+    if (b0 >= b1) return;
+    bin_starts(s, sh, running, wsum);
+    // (the place of a bin the block has no contact of is not set, and not used)
+    for (uint32_t k = threadIdx.x; k < sh.coarse; k += kBucketThreads)
+        running[k] += s.boff[(size_t)k * blk.count() + blk.id()];
     for (unsigned long long t0 = b0; t0 < b1; t0 += kBucketTile) {
         const uint32_t tn = (uint32_t)min((unsigned long long)kBucketTile, b1 - t0);
         for (uint32_t k = threadIdx.x; k < nb; k += kBucketThreads) hist[k] = 0;
@@ -3374,8 +3320,7 @@ __device__ __forceinline__ void bucket_scatter_body(const DevState s, const P bl
         }
 #pragma unroll
         for (int q = 0; q < kBucketTile / kBucketThreads; q++) {
-            const uint32_t i = threadIdx.x + q * kBucketThreads;
-            rk[q] = i < tn ? atomicAdd(&hist[coarse_bin(sh, keys[q])], 1u) : 0u;
+            rk[q] = keys[q] != kEmptyKey ? atomicAdd(&hist[coarse_bin(sh, keys[q])], 1u) : 0u;
         }
         __syncthreads();
         // exclusive scan of the tile histogram (nb <= 1025 bins, kPer per thread)
@@ -3405,14 +3350,14 @@ __device__ __forceinline__ void bucket_scatter_body(const DevState s, const P bl
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < kBucketTile / kBucketThreads; q++) {
-            uint32_t i = threadIdx.x + q * kBucketThreads;
-            if (i < tn) tile[start[coarse_bin(sh, keys[q])] + rk[q]] = keys[q];
+            if (keys[q] != kEmptyKey) tile[start[coarse_bin(sh, keys[q])] + rk[q]] = keys[q];
         }
         __syncthreads();
-        for (uint32_t p = threadIdx.x; p < tn; p += kBucketThreads) {
-            unsigned long long key = tile[p];
-            uint32_t b = coarse_bin(sh, key);
-            if (b < sh.coarse) out[running[b] + (p - start[b])] = key;
+        // (the empty slots' bin, the last, is empty: the tile's contacts end at its start)
+        for (uint32_t p = threadIdx.x; p < start[sh.coarse]; p += kBucketThreads) {
+            const unsigned long long key = tile[p];
+            const uint32_t b = coarse_bin(sh, key);
+            out[running[b] + (p - start[b])] = key;
         }
         __syncthreads();
         for (uint32_t k = threadIdx.x; k < nb; k += kBucketThreads) running[k] += hist[k];
@@ -3460,74 +3405,95 @@ __device__ __forceinline__ uint32_t block_scan_bins(uint32_t *bins, uint32_t nbi
     return total;
 }
 
+struct FineLds {
+    unsigned long long tile[kFineTile];
+    uint32_t thist[kMaxFine], tstart[kMaxFine], gcur[kMaxFine];
+    uint32_t wsum[kBucketThreads / 64];
+    uint32_t start[kMaxCoarse + 1];
+};
+
 template <class P>
 __device__ __forceinline__ void bucket_fine_body(const DevState s, const P blk)
 {
-    __shared__ unsigned long long tile[kFineTile];
-    __shared__ uint32_t thist[kMaxFine], tstart[kMaxFine], gcur[kMaxFine];
-    __shared__ uint32_t wsum[kBucketThreads / 64];
-    const uint32_t G1 = s.bucket_blocks;
+    __shared__ FineLds L;
     const TableShape sh = table_shape(s);
-    const uint32_t nf = 1u << sh.lo_bits;
+    const unsigned long long n = min(s.ctr->n_clist, s.clist_cap);
     unsigned long long *out = s.tp->tab_cur.keys;
     uint32_t *rstart = s.tp->tab_cur.rstart;
-    for (uint32_t c = blk.id(); c < sh.coarse; c += blk.count()) {
-        const uint32_t seg0 = s.boff[(size_t)c * G1], seg1 = s.boff[(size_t)(c + 1) * G1];
-        for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) thist[k] = 0;
-        __syncthreads();
-        for (uint32_t i0 = seg0 + threadIdx.x; i0 < seg1; i0 += 4 * kBucketThreads) {
-            unsigned long long key[4];
+    // a list of one tile: the regions are the bins of one segment, read where
+    // the join left it and written back in place (a tile is held whole
+    // before it is written)
+    const bool one = one_tile(n, sh);
+    if (one && blk.id() != 0) return;
+    const uint32_t nf = one ? 1u << sh.bits : 1u << sh.lo_bits;
+    const uint32_t nseg = one ? 1u : sh.coarse;
+    const unsigned long long *in = one ? contact_out(s) : s.clist2;
+    uint32_t total = 0;
+    if (!one) {
+        bin_starts(s, sh, L.start, L.wsum);
+        total = L.start[sh.coarse];
+    }
+    constexpr int kPer = kFineTile / kBucketThreads;
+    for (uint32_t c = blk.id(); c < nseg; c += blk.count()) {
+        const uint32_t seg0 = one ? 0u : L.start[c], seg1 = one ? (uint32_t)n : L.start[c + 1];
+        if (!one) {   // (a single tile's own histogram gives the regions' starts)
+            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) L.thist[k] = 0;
+            __syncthreads();
+            for (uint32_t i0 = seg0 + threadIdx.x; i0 < seg1; i0 += 4 * kBucketThreads) {
+                unsigned long long key[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) key[q] = i0 + q * kBucketThreads < seg1 ? s.clist2[i0 + q * kBucketThreads] : 0ull;
+                for (int q = 0; q < 4; q++) key[q] = i0 + q * kBucketThreads < seg1 ? in[i0 + q * kBucketThreads] : 0ull;
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (i0 + q * kBucketThreads < seg1) atomicAdd(&thist[region_of(key[q] & kKeyBits, sh.bits) & (nf - 1)], 1u);
+                for (int q = 0; q < 4; q++)
+                    if (i0 + q * kBucketThreads < seg1)
+                        atomicAdd(&L.thist[region_of(key[q] & kKeyBits, sh.bits) & (nf - 1)], 1u);
+            }
+            __syncthreads();
+            block_scan_bins(L.thist, nf, L.gcur, seg0, L.wsum);
+            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) rstart[(size_t)c * nf + k] = L.gcur[k];
+            __syncthreads();
         }
-        __syncthreads();
-        block_scan_bins(thist, nf, gcur, seg0, wsum);
-        for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) rstart[(size_t)c * nf + k] = gcur[k];
-        __syncthreads();
-        for (uint32_t t0 = seg0; t0 < seg1; t0 += kFineTile) {
+        for (uint32_t t0 = seg0; t0 < seg1 || (one && t0 == 0); t0 += kFineTile) {
             const uint32_t tn = min((uint32_t)kFineTile, seg1 - t0);
-            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) thist[k] = 0;
+            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) L.thist[k] = 0;
             __syncthreads();
-            unsigned long long keys[kFineTile / kBucketThreads];
-            uint32_t fb[kFineTile / kBucketThreads], rk[kFineTile / kBucketThreads];
+            unsigned long long keys[kPer];
+            uint32_t fb[kPer], rk[kPer];
 #pragma unroll
-            for (int q = 0; q < kFineTile / kBucketThreads; q++) {   // every load before the first atomic
+            for (int q = 0; q < kPer; q++) {   // every load before the first atomic
                 const uint32_t i = threadIdx.x + q * kBucketThreads;
-                keys[q] = i < tn ? s.clist2[t0 + i] : 0ull;
+                keys[q] = i < tn ? in[t0 + i] : kEmptyKey;
             }
 #pragma unroll
-            for (int q = 0; q < kFineTile / kBucketThreads; q++) {
-                const uint32_t i = threadIdx.x + q * kBucketThreads;
+            for (int q = 0; q < kPer; q++) {
                 fb[q] = region_of(keys[q] & kKeyBits, sh.bits) & (nf - 1);
-                rk[q] = i < tn ? atomicAdd(&thist[fb[q]], 1u) : 0u;   // its rank in the region
+                rk[q] = keys[q] != kEmptyKey ? atomicAdd(&L.thist[fb[q]], 1u) : 0u;   // its rank in the region
             }
             __syncthreads();
-            block_scan_bins(thist, nf, tstart, 0, wsum);
+            const uint32_t held = block_scan_bins(L.thist, nf, L.tstart, 0, L.wsum);
+            if (one) {
+                total = held;
+                for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) L.gcur[k] = rstart[k] = L.tstart[k];
+            }
             __syncthreads();
 #pragma unroll
-            for (int q = 0; q < kFineTile / kBucketThreads; q++) {
-                const uint32_t i = threadIdx.x + q * kBucketThreads;
-                if (i < tn) tile[tstart[fb[q]] + rk[q]] = keys[q];
-            }
+            for (int q = 0; q < kPer; q++)
+                if (keys[q] != kEmptyKey) L.tile[L.tstart[fb[q]] + rk[q]] = keys[q];
             __syncthreads();
-            for (uint32_t p = threadIdx.x; p < tn; p += kBucketThreads) {
-                const unsigned long long key = tile[p];
+            for (uint32_t p = threadIdx.x; p < held; p += kBucketThreads) {
+                const unsigned long long key = L.tile[p];
                 const uint32_t f = region_of(key & kKeyBits, sh.bits) & (nf - 1);
-                out[gcur[f] + (p - tstart[f])] = key;
+                out[L.gcur[f] + (p - L.tstart[f])] = key;
             }
             __syncthreads();
-            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) gcur[k] += thist[k];
+            for (uint32_t k = threadIdx.x; k < nf; k += kBucketThreads) L.gcur[k] += L.thist[k];
             __syncthreads();
         }
     }
     if (blk.id() == 0 && threadIdx.x == 0) {
         // the generation's entry count and region bits, where the next tick
         // (and the readers of a generation) find them whatever its shape
-        const uint32_t total = s.boff[(size_t)sh.coarse * G1];
-        rstart[(size_t)sh.coarse * nf] = total;
+        rstart[1u << sh.bits] = total;
         rstart[s.rs_total] = total;
         rstart[s.rs_total + 1] = sh.bits;
         s.ctr->tab_bits = sh.bits;
@@ -3991,12 +3957,12 @@ double sqrt_threshold(double r)
 
 enum KernelId {
     K_BEGIN_TICK, K_ASSIGN, K_SCAN_OBJECTS, K_PLACE, K_SCAN_UNITS, K_UNIT_SCATTER, K_JOIN, K_BUCKET_COUNT,
-    K_SCAN_REDUCE, K_SCAN_TOP, K_SCAN_WRITE, K_BUCKET_SCATTER, K_BUCKET_FINE, K_POS32, K_TABLE, K_COLLECT, K_SCHEMA,
+    K_BUCKET_SCATTER, K_BUCKET_FINE, K_POS32, K_TABLE, K_COLLECT, K_SCHEMA,
     K_GRID_CELLS, K_GRID_PYRAMID, K_GRID_TOP, K_GRID_FINE_ZERO, K_GRID_FINE, K_GRID_LEVEL, K_COUNT
 };
 const char *const kKernelNames[K_COUNT] = {
     "k_begin_tick", "k_assign", "k_scan_objects", "k_place", "k_scan_units", "k_unit_scatter", "k_join",
-    "k_bucket_count", "k_scan_reduce", "k_scan_top", "k_scan_write", "k_bucket_scatter", "k_bucket_fine", "k_pos32",
+    "k_bucket_count", "k_bucket_scatter", "k_bucket_fine", "k_pos32",
     "k_table", "k_collect", "k_schema", "k_grid_cells", "k_grid_pyramid", "k_grid_top", "k_grid_fine_zero",
     "k_grid_fine", "k_grid_level"};
 
@@ -4291,28 +4257,6 @@ void step(const Seq &q, int id, B blocks, S single, F fused)
         [&](hipStream_t st_, uint32_t g_, glint_ctx &c) { k_##name<<<g_, threads, 0, st_>>>(c.s); },     \
         [&](hipStream_t st_, uint32_t g_, const Many &m_) { kf_##name<<<g_, threads, 0, st_>>>(m_); })
 
-// The three kernels that scan the region bins.
-void step_scan_bins(const Seq &q)
-{
-    auto nb = [](const glint_ctx &c) -> uint32_t { return scan_blocks_for(bins_length(c.s)); };
-    step(
-        q, K_SCAN_REDUCE, nb,
-        [&](hipStream_t st, uint32_t g, glint_ctx &c) {
-            k_scan_reduce<<<g, kBlock, 0, st>>>(c.s.bcount, bins_length(c.s), c.s.block_sums);
-        },
-        [&](hipStream_t st, uint32_t g, const Many &m) { kf_scan_reduce<<<g, kBlock, 0, st>>>(m); });
-    step(
-        q, K_SCAN_TOP, [](const glint_ctx &) -> uint32_t { return 1; },
-        [&](hipStream_t st, uint32_t, glint_ctx &c) { k_scan_top<<<1, kBlock, 0, st>>>(c.s.block_sums, nb(c)); },
-        [&](hipStream_t st, uint32_t g, const Many &m) { kf_scan_top<<<g, kBlock, 0, st>>>(m); });
-    step(
-        q, K_SCAN_WRITE, nb,
-        [&](hipStream_t st, uint32_t g, glint_ctx &c) {
-            k_scan_write<<<g, kBlock, 0, st>>>(c.s.bcount, bins_length(c.s), c.s.block_sums, c.s.boff);
-        },
-        [&](hipStream_t st, uint32_t g, const Many &m) { kf_scan_write_bins<<<g, kBlock, 0, st>>>(m); });
-}
-
 // The tree of this tick's positions (GLINT_SCHEMA_GRID_REBUILD), before the
 // assignment: a fixed sequence of launches.
 void enqueue_grid_rebuild(const Seq &q)
@@ -4381,8 +4325,7 @@ void enqueue_refine(const Seq &q)
     // group the tick's contacts by table region
     // (the table's shape is decided on the device from the tick's stored
     // contacts; launch sizes cover the largest shape)
-    GLINT_STEP(q, K_BUCKET_COUNT, kBlock, c.s.bucket_blocks, bucket_count);
-    step_scan_bins(q);
+    GLINT_STEP(q, K_BUCKET_COUNT, kBucketThreads, c.s.bucket_blocks, bucket_count);
     GLINT_STEP(q, K_BUCKET_SCATTER, kBucketThreads, c.s.bucket_blocks, bucket_scatter);
     GLINT_STEP(q, K_BUCKET_FINE, kBucketThreads, c.fine_grid, bucket_fine);
 }
@@ -4753,9 +4696,11 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
         s.coarse_max = 1u << (s.rbits_max - lo);
         s.rs_total = 1u << s.rbits_max;
         // coarse-pass workgroups: one per 4 tiles of the configured
-        // contacts, a power of two from 16 to 1024
+        // contacts, a power of two from 16 to 256 (one fills a CU's LDS, and
+        // each adds its counts to every bin's total: 10M objects in hotspots
+        // take 51.5 ms for 8 ticks with 256, 52.1 with 512 or 1024)
         uint32_t bb = 16;
-        while (bb < 1024 && (uint64_t)bb * 4 * kBucketTile < contacts) bb *= 2;
+        while (bb < 256 && (uint64_t)bb * 4 * kBucketTile < contacts) bb *= 2;
         s.bucket_blocks = bb;
         // the persistent passes get the workgroups of the configured shape
         // (at least 256 table regions and 64 bins when the shape can grow
@@ -4767,8 +4712,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
         c->fine_grid = std::min<uint32_t>(s.coarse_max, std::max<uint32_t>(fine_min, 64));
     }
     c->scan_blocks = (uint32_t)((node_cap + kScanTile - 1) / kScanTile);
-    const uint64_t nbc = (uint64_t)(s.coarse_max + 1) * s.bucket_blocks;
-    const uint32_t sum_blocks = (uint32_t)((nbc + kScanTile - 1) / kScanTile);
+    const uint64_t nbc = (uint64_t)s.coarse_max * s.bucket_blocks;
 
     glint_status st = GLINT_OK;
 #define ALLOC(p, n)                          \
@@ -4781,8 +4725,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
     ALLOC(s.free_stack, node_cap);
     ALLOC(s.count, node_cap);
     ALLOC(s.offset, node_cap);
-    ALLOC(s.block_sums, sum_blocks);
-    ALLOC(s.bcount, nbc);
+    ALLOC(s.bins, (uint64_t)s.coarse_max * kBinStride);
     ALLOC(s.boff, nbc);
     ALLOC(s.clist2, s.clist_cap);
     ALLOC(s.split_list, node_cap);

@@ -213,7 +213,6 @@ struct DevState {
     int32_t *free_stack;
     uint32_t *count;
     uint32_t *offset;
-    uint32_t *block_sums;
     uint32_t *split_list;
     uint32_t *merge_list;
     uint32_t *leaf_list;
@@ -255,8 +254,8 @@ struct DevState {
     float *pfy;             // (NaN beyond pf_lim: left to the FP64 test)
     glint_meeting *meet;
     unsigned long long *clist2;    // bucketing buffer (the join's output when there is one pass)
-    uint32_t *bcount;              // coarse-bin counts per bucketing block
-    uint32_t *boff;                // their exclusive offsets
+    uint32_t *bins;                // contacts per coarse bin, a line each
+    uint32_t *boff;                // per coarse bin and bucketing block: its place in the bin
     uint32_t rbits_min;            // log2(regions) of the configured table: the fewest a tick uses
     uint32_t rbits_max;            // the most a tick can need (its stored contacts are below clist_cap)
     uint32_t coarse_max;           // first-pass bins at rbits_max
