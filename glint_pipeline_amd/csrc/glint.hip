@@ -1634,11 +1634,11 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t *to
 }
 
 // The children of a node as the lookup sees them: the four child nodes are
-// read together; accepted leaves are passed to take(leaf) when `takes`, and
-// the mask of branch children within r is returned.
+// read together; accepted leaves are passed to take(leaf), and the mask of
+// branch children within r is returned.
 template <bool GEO, class Take>
 __device__ __forceinline__ uint32_t lookup_children(const DevState &s, uint4 ids, double x, double y, double f,
-                                                    uint32_t own, bool takes, Take &&take)
+                                                    uint32_t own, Take &&take)
 {
     const Node n0 = s.nodes[ids.x], n1 = s.nodes[ids.y], n2 = s.nodes[ids.z], n3 = s.nodes[ids.w];
     uint32_t desc = 0;
@@ -1646,7 +1646,7 @@ __device__ __forceinline__ uint32_t lookup_children(const DevState &s, uint4 ids
         if (!(GEO ? box_within_geo(cn, x, y, s.t64, f) : box_within(cn, x, y, s.t64))) return;
         if (cn.child[0] != kLeafTag) {
             desc |= bit;
-        } else if (takes && (s.complete ? (c != own) : (y < cn.ly || (y < cn.hy && x < cn.lx)))) {
+        } else if ((s.complete ? (c != own) : (y < cn.ly || (y < cn.hy && x < cn.lx)))) {
             take(c);
         }
     };
@@ -1657,52 +1657,77 @@ __device__ __forceinline__ uint32_t lookup_children(const DevState &s, uint4 ids
     return desc;
 }
 
-// lookup_rec (filter.cpp:130-152) below node `from`: every leaf within r of
-// (x, y) that the top/right rule accepts (in complete mode every leaf within
-// r other than `own`) is passed to take(leaf).  A depth-first walk without a
-// stack in memory: the branch children still to visit at each of the first
-// 16 levels below `from` are kept as 4-bit masks in one 64-bit register, and
-// the walk climbs back through the parent links (deeper levels recompute
-// their mask from the children), so nothing sits in scratch memory.
-// GEO: geography, f the degrees of longitude per metre at y.
+// lookup_rec (filter.cpp:130-152) below every lane's node `from`: each leaf
+// within r of the lane's object that the top/right rule accepts (in complete
+// mode every leaf within r other than its own) is passed to take(lane, leaf),
+// in no particular order.
+// The objects of a wave need from one to some twenty visits of a branch and
+// its children, each a wait for memory, so the wave shares them: the branches
+// to visit, of any of its objects, are kept on one stack in LDS and taken 64
+// at a time.  (A walk of its own per lane lasted as long as the longest: 28 us
+// of the 30 that 4300 lookups of 100k objects took.)
+// Taking fewer when the stack is nearly full keeps it within its bounds: 64
+// visits grow it by at most three each up to kWalkStack - kWalkRoom, and one
+// at a time, depth first, it needs three per level of the tree more.
+constexpr uint32_t kWalkStack = 512;
+constexpr uint32_t kWalkRoom = 192;   // three per level, at most 64 levels
+
+struct WalkLds {
+    uint32_t node[kWalkStack];
+    uint8_t who[kWalkStack];
+    double2 pos[64];             // the lanes' objects
+    double f[64];                // geography: degrees of longitude per metre there
+    uint32_t own[64];            // their leaves
+    uint32_t found[64];          // leaves accepted
+    uint32_t cand[64][3];        // the first three of them
+    uint32_t pid[64];            // written with their units
+    uint4 aux[64];
+    unsigned long long at[64];   // places of the units of objects with more than three
+};
+
 template <bool GEO, class Take>
-__device__ __forceinline__ void lookup_walk(const DevState &s, double x, double y, double f, uint32_t from,
-                                            uint32_t own, Take &&take)
+__device__ __forceinline__ void wave_walk(const DevState &s, WalkLds &L, bool valid, uint32_t from, Take &&take)
 {
-    uint32_t node = from;
-    uint4 ids = node_children(s.nodes, from);
-    uint32_t desc = lookup_children<GEO>(s, ids, x, y, f, own, true, take);
-    unsigned long long masks = 0;   // level d (< 16): masks >> 4d
-    uint32_t depth = 0;             // of `node` below `from`
-    for (;;) {
-        if (desc) {
-            const uint32_t ci = __builtin_ctz(desc);
-            if (depth < 16) {
-                const unsigned long long rest = desc & ~((2u << ci) - 1u);
-                masks = (masks & ~(0xFull << (4 * depth))) | (rest << (4 * depth));
+    const uint32_t lane = lane_id();
+    unsigned long long m = __builtin_amdgcn_ballot_w64(valid);
+    uint32_t n = (uint32_t)__popcll(m);
+    auto push = [&](unsigned long long mask, uint32_t base, uint32_t node, uint32_t who) {
+        if (!__builtin_amdgcn_inverse_ballot_w64(mask)) return;
+        const uint32_t at =
+            base + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+        L.node[at] = node;
+        L.who[at] = (uint8_t)who;
+    };
+    push(m, 0u, from, lane);
+    while (n) {
+        wave_sync();
+        const uint32_t room = n + kWalkRoom < kWalkStack ? (kWalkStack - kWalkRoom - n) / 3 : 0u;
+        const uint32_t take_n = min(min(n, 64u), max(room, 1u));
+        n -= take_n;
+        uint32_t desc = 0, who = 0;
+        uint4 ids = make_uint4(0u, 0u, 0u, 0u);
+        if (lane < take_n) {
+            ids = node_children(s.nodes, L.node[n + lane]);
+            who = L.who[n + lane];
+        }
+        wave_sync();   // (the entries taken may be written over)
+        if (lane < take_n) {
+            const double2 p = L.pos[who];
+            desc = lookup_children<GEO>(s, ids, p.x, p.y, GEO ? L.f[who] : 0.0, L.own[who],
+                                        [&](uint32_t leaf) { take(who, leaf); });
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < 4; b++) {
+            m = __builtin_amdgcn_ballot_w64(((desc >> b) & 1u) != 0u);
+            if (n + (uint32_t)__popcll(m) > kWalkStack) {   // a tree of more than 64 levels
+                if (lane == 0) atomicOr(&s.ctr->error, kErrStack);
+                m = 0;
             }
-            node = pick_child(ids, (int)ci);
-            depth++;
-            ids = node_children(s.nodes, node);
-            desc = lookup_children<GEO>(s, ids, x, y, f, own, true, take);
-            continue;
+            push(m, n, b == 0 ? ids.x : b == 1 ? ids.y : b == 2 ? ids.z : ids.w, who);
+            n += (uint32_t)__popcll(m);
         }
-        if (node == from) break;
-        const uint32_t p = s.parent[node];
-        if (p >= s.node_cap) {   // not reached: every node below `from` has its parent
-            atomicOr(&s.ctr->error, kErrStack);
-            break;
-        }
-        depth--;
-        ids = node_children(s.nodes, p);
-        if (depth < 16) {
-            desc = (uint32_t)(masks >> (4 * depth)) & 0xFu;
-        } else {
-            const uint32_t ci = ids.x == node ? 0u : (ids.y == node ? 1u : (ids.z == node ? 2u : 3u));
-            desc = lookup_children<GEO>(s, ids, x, y, f, own, false, take) & ~((2u << ci) - 1u);
-        }
-        node = p;
     }
+    wave_sync();
 }
 
 // The lookup from last_valid for every border object.  Each unit (object,
@@ -1712,21 +1737,25 @@ __device__ __forceinline__ void lookup_walk(const DevState &s, double x, double 
 // Objects with up to three candidates (nearly all) write their units from
 // registers after one atomic per workgroup; the others walk a second time.
 // Counting a wave's target leaves together and one reservation per workgroup
-// took it from 0.74 to 0.52 ms at 10M objects in hotspots (3.1M lookups); at
-// 100k objects (29 us) it is one chain of dependent node reads.
+// took it from 0.74 to 0.52 ms at 10M objects in hotspots (3.1M lookups), the
+// walk shared by the wave its launch (with the scatter) from 29 to 19 us at
+// 100k objects and from 56 to 32 at 1M uniform ones, where it is still a chain
+// of some ten node reads.
 template <bool GEO, class P>
 __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
 {
     const uint32_t nb = s.ctr->n_border;
     __shared__ uint32_t wunits[2][kBlock / 64];
     __shared__ unsigned long long unit_at[2];
+    __shared__ WalkLds walk[kBlock / 64];
+    WalkLds &L = walk[threadIdx.x / 64];
+    const uint32_t lane = lane_id();
     uint32_t turn = 0;
     for (uint32_t base = blk.id() * blockDim.x; base < nb; base += blk.count() * blockDim.x, turn ^= 1) {
         const uint32_t k = base + threadIdx.x;
         uint32_t total = 0;
         uint32_t f0 = kNone, f1 = kNone, f2 = kNone;
         uint32_t pid = 0, lv = 0, own = 0, pleaf = kNone, prevk = kNone, pos = 0;
-        double x = 0.0, y = 0.0, f = 0.0;
         if (k < nb) {
             const BorderObj b = s.border[k];
             pid = s.order[b.k];
@@ -1736,16 +1765,21 @@ __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
             const double2 p = s.ord_xy[b.k];
             lv = b.lv & ~kBorderOrdered;
             prevk = (b.lv & kBorderOrdered) ? b.k : kNone;
-            x = p.x;
-            y = p.y;
-            if (GEO) f = deg_per_meter_lon(y);
             pos += s.offset[own];
-            lookup_walk<GEO>(s, x, y, f, lv, own, [&](uint32_t c) {
-                f0 = total == 0 ? c : f0;
-                f1 = total == 1 ? c : f1;
-                f2 = total == 2 ? c : f2;
-                total++;
-            });
+            L.pos[lane] = p;
+            if (GEO) L.f[lane] = deg_per_meter_lon(p.y);
+            L.own[lane] = own;
+        }
+        L.found[lane] = 0;
+        wave_walk<GEO>(s, L, k < nb, lv, [&](uint32_t who, uint32_t leaf) {
+            const uint32_t slot = atomicAdd(&L.found[who], 1u);
+            if (slot < 3) L.cand[who][slot] = leaf;
+        });
+        if (k < nb) {
+            total = L.found[lane];
+            f0 = total > 0 ? L.cand[lane][0] : kNone;
+            f1 = total > 1 ? L.cand[lane][1] : kNone;
+            f2 = total > 2 ? L.cand[lane][2] : kNone;
             if (!s.store_all) s.tp->cand[pos] = make_uint4(f0, f1, total > 3 ? kCandOverflow : f2, s.tp->tick);
         }
         // one atomic per workgroup reserves the units of the lists of up to
@@ -1773,22 +1807,29 @@ __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
         unsigned long long u = unit_at[turn] + before + wex;
         // what the join's border rows need of the object, beside each unit
         const uint4 aux = make_uint4(own | (total > 3 ? 0x80000000u : 0u), pleaf, prevk, pos);
-        auto write = [&](uint32_t c, uint32_t rank) {
-            if (u < s.unit_cap) {
-                s.units[u] = make_uint2(pid, c);
-                s.uaux[u] = aux;
-                s.urank[u] = rank;
+        auto write = [&](unsigned long long at, uint32_t object, const uint4 &beside, uint32_t c, uint32_t rank) {
+            if (at < s.unit_cap) {
+                s.units[at] = make_uint2(object, c);
+                s.uaux[at] = beside;
+                s.urank[at] = rank;
             } else {
                 atomicOr(&s.ctr->error, kErrUnitCap);
             }
-            u++;
         };
-        if (nc > 0) write(f0, r0);
-        if (nc > 1) write(f1, r1);
-        if (nc > 2) write(f2, r2);
-        if (total > 3) {
-            u = atomicAdd(&s.ctr->n_units, (unsigned long long)total);
-            lookup_walk<GEO>(s, x, y, f, lv, own, [&](uint32_t c) { write(c, atomicAdd(&s.ucount[c], 1u)); });
+        if (nc > 0) write(u, pid, aux, f0, r0);
+        if (nc > 1) write(u + 1, pid, aux, f1, r1);
+        if (nc > 2) write(u + 2, pid, aux, f2, r2);
+        if (__builtin_amdgcn_ballot_w64(total > 3)) {   // (the same on every lane)
+            if (total > 3) {
+                L.at[lane] = atomicAdd(&s.ctr->n_units, (unsigned long long)total);
+                L.pid[lane] = pid;
+                L.aux[lane] = aux;
+            }
+            L.found[lane] = 0;
+            wave_walk<GEO>(s, L, total > 3, lv, [&](uint32_t who, uint32_t leaf) {
+                write(L.at[who] + atomicAdd(&L.found[who], 1u), L.pid[who], L.aux[who], leaf,
+                      atomicAdd(&s.ucount[leaf], 1u));
+            });
         }
     }
 }
@@ -4130,7 +4171,7 @@ glint_status status_from_flags(glint_ctx *c, uint32_t f)
         return GLINT_ERR_TABLE_FULL;
     }
     if (f & kErrStack) {
-        c->err = "inconsistent quadtree (a node without its parent link)";
+        c->err = "quadtree too deep for the lookup";
         return GLINT_ERR_HIP;
     }
     if (f & kErrUnitCap) {

@@ -217,7 +217,7 @@ struct DevState {
     uint32_t *merge_list;
     uint32_t *leaf_list;
     uint32_t *sparse_list;  // leaves the join gives to one wave each
-    uint32_t *parent;       // per node: its parent (kNone for the root), for stackless tree walks
+    uint32_t *parent;       // per node: its parent (kNone for the root), for descents that start at the last leaf
     double4 *region;        // per node: the points the descent sends into it, (x.lo, x.hi] x (y.lo, y.hi]
     uint32_t incremental;   // objects are placed from their leaf of the tick before (not with the grid rebuild)
     uint32_t pad_inc_;
