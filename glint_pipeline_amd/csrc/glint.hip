@@ -50,7 +50,8 @@ constexpr uint32_t kMaxRegionBits = 21;             // at most 2^21 regions (coa
 constexpr int kBucketThreads = 1024;                // workgroup of the two bucketing passes
 constexpr int kBucketTile = 16384;                  // contacts per LDS tile of the coarse pass (128 KB)
 constexpr int kFineTile = 12288;                    // contacts per LDS tile of the fine pass (96 KB)
-constexpr uint32_t kMaxCoarse = 1024;               // coarse bins of pass 1
+constexpr uint32_t kMaxCoarse = 1024;               // coarse bins of pass 1 at most
+constexpr uint32_t kCoarseBits = 8;                 // 256 of them unless pass 2 would have more than kMaxFine
 constexpr uint32_t kBinStride = 32;                 // words between their totals (a line each)
 constexpr uint32_t kMaxFine = 2048;                 // fine bins of pass 2
 constexpr int kBorderStage = 512;                   // staged border objects per wave (assign)
@@ -1937,13 +1938,28 @@ struct TableShape {
     uint32_t bits, lo_bits, coarse;
 };
 
+// Coarse bins of 2^bits regions, as a power of two: 256, as many as there are
+// CUs for pass 2 (a workgroup fills a CU's LDS), fewer only when there are
+// fewer regions and more only when pass 2 could not split the rest.  Pass 1
+// then writes runs of 64 contacts of a tile, pass 2 of 12288 over the regions
+// of a bin.  128 / 256 / 512 / 1024 bins (us of 8 ticks): 10M objects in
+// hotspots, 2^17 regions, 53200 / 51200 / 51200 / 51600 (pass 1 takes 400, 460
+// and 535 us a tick, pass 2 655, 590 and 575); 2M with the grid rebuild 10900 /
+// 10740 / 10790 / 10960; 400k in hotspots with key-value flush 4720 / 4750 /
+// 4820 / 4960.
+__host__ __device__ inline uint32_t coarse_bits(uint32_t bits)
+{
+    static_assert(kMaxFine == 2048 && kMaxRegionBits - 11 <= 10, "2^11 fine bins, at most 2^10 coarse ones");
+    return bits <= kCoarseBits ? bits : bits > kCoarseBits + 11 ? bits - 11 : kCoarseBits;
+}
+
 __device__ __forceinline__ TableShape table_shape(const DevState &s, unsigned long long n)
 {
     uint32_t b = s.rbits_min;
     while (b < s.rbits_max && ((unsigned long long)kRegionFill << b) < n) b++;
     TableShape t;
     t.bits = b;
-    t.lo_bits = b > 10 ? b - 10 : 0;
+    t.lo_bits = b - coarse_bits(b);
     t.coarse = 1u << (b - t.lo_bits);
     return t;
 }
@@ -3229,7 +3245,7 @@ __global__ __launch_bounds__(kBlock, 4) void kf_join(const Many m)   // (4 waves
 //
 // Two passes group the contact list by region.  Pass 1 (k_bucket_count,
 // k_bucket_scatter) splits it by the high bits of the region index into
-// at most 1024 coarse bins; each block sorts 16384-entry tiles in LDS so its
+// 2^coarse_bits coarse bins; each block sorts 16384-entry tiles in LDS so its
 // writes form runs.  Pass 2 (k_bucket_fine) splits every coarse bin by the low
 // bits with one workgroup per bin and records the first contact of every region.
 // The counting pass adds every block's counts to the bins' totals, a line
@@ -4733,8 +4749,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
         while (most < kMaxRegionBits && ((uint64_t)kRegionFill << most) < s.clist_cap) most++;
         s.rbits_min = std::min<uint32_t>(bits, kMaxRegionBits);
         s.rbits_max = std::max(s.rbits_min, most);
-        const uint32_t lo = s.rbits_max > 10 ? s.rbits_max - 10 : 0;
-        s.coarse_max = 1u << (s.rbits_max - lo);
+        s.coarse_max = 1u << coarse_bits(s.rbits_max);
         s.rs_total = 1u << s.rbits_max;
         // coarse-pass workgroups: one per 4 tiles of the configured
         // contacts, a power of two from 16 to 256 (one fills a CU's LDS, and
@@ -4748,8 +4763,7 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
         // that far); a tick whose table grows past it loops over the rest
         c->table_grid = std::min<uint32_t>(
             std::max<uint32_t>(1u << s.rbits_min, std::min<uint32_t>(1u << s.rbits_max, 256)), 4096);
-        // (a shape of b bits has min(2^b, 1024) coarse bins)
-        const uint32_t fine_min = 1u << std::min<uint32_t>(s.rbits_min, 10);
+        const uint32_t fine_min = 1u << coarse_bits(s.rbits_min);
         c->fine_grid = std::min<uint32_t>(s.coarse_max, std::max<uint32_t>(fine_min, 64));
     }
     c->scan_blocks = (uint32_t)((node_cap + kScanTile - 1) / kScanTile);

@@ -26,3 +26,16 @@ def test_lists_around_one_tile(crowd, buckets):
     for record in (False, True):
         run_positions_parity(xys, (0.0, 0.0, 800.0, 800.0), grid_capacity=300, min_meet=2, num_meeting_buckets=buckets,
                              contact_capacity=1 << 16, record_contacts=record)
+
+
+@pytest.mark.parametrize("bits", [7, 8, 9, 11, 12, 19, 20, 21])
+def test_numbers_of_regions(bits):
+    """2^bits regions: 256 coarse bins, fewer with fewer regions, more past
+    2^19 of them; 26335 pairs, more than one workgroup takes whole."""
+    print(f"[bucketing] 2^{bits} regions", flush=True)
+    rng = np.random.default_rng(bits)
+    xys = [(400.0 + rng.uniform(0.0, 1.0, (230, 2)) + (np.arange(230)[:, None] % 7 == t) * 30.0).reshape(-1)
+           for t in range(7)]
+    for record in (False, True):
+        run_positions_parity(xys, (0.0, 0.0, 800.0, 800.0), grid_capacity=300, min_meet=2,
+                             num_meeting_buckets=1 << (bits + 11), contact_capacity=1 << 16, record_contacts=record)
