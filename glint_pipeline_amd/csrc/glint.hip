@@ -5309,6 +5309,13 @@ glint_status glint_contacts(glint_ctx *c, uint64_t *out, uint64_t cap, uint64_t 
     glint_status st = read_counters(c);
     if (st) return st;
     if (c->h_ctr->error) return status_from_flags(c, c->h_ctr->error);
+    // The number alone, which callers ask for first to size their buffer, is
+    // known once the table has found the second copies: no copy and no sort
+    // (stage calls with contacts read, 3000 objects: 325 -> 270 us a tick).
+    if (!out && c->evaluated) {
+        *n_out = c->h_ctr->n_contacts - c->h_ctr->n_dup;
+        return GLINT_OK;
+    }
     // the tick's bucketed contact list holds exactly n_contacts entries
     const uint64_t n = std::min<uint64_t>(c->h_ctr->n_contacts, c->s.clist_cap);
     // after evaluate the tick's list is the previous generation
