@@ -73,6 +73,10 @@ constexpr uint32_t kSparseMax = 512;                // most objects of a leaf jo
 // 8.6, 8.5, 8.6 and 9.2 ms; 3000 objects at 0.012 a square metre 0.42, 0.40,
 // 0.40 and 0.39 ms.
 constexpr double kSparseDensity = 0.25;
+// and fewer reaches across than its single-precision offsets in reaches, and
+// their squares, can hold (a reach of 1e-40, or a box 1e39 metres wide: their
+// infinities had lost contacts).
+constexpr double kSparseSides = 1e12;
 
 // ------------------------------------------------------------ predicates
 
@@ -1542,7 +1546,9 @@ __device__ __forceinline__ void scan_units_body(const DevState s, const P blk)
         if (cnt <= kSparseMax) {
             const double2 lo = reinterpret_cast<const double2 *>(s.nodes + n)[1], hi = node_high(s.nodes, n);
             const double2 r = sparse_reach(s, lo.y, hi.y);
-            if ((double)cnt * r.x * r.y <= kSparseDensity * (hi.x - lo.x) * (hi.y - lo.y) && r.x > 0.0) kind[k] = 3;
+            const double w = hi.x - lo.x, h = hi.y - lo.y;   // (r.x is 0 where a leaf is left to the tiles)
+            if ((double)cnt * r.x * r.y <= kSparseDensity * w * h && w < kSparseSides * r.x && h < kSparseSides * r.y)
+                kind[k] = 3;
         }
         listed += kind[k] == 1 ? 1u : kind[k] == 2 ? 0x10000u : 0u;
         sparse += kind[k] == 3;
