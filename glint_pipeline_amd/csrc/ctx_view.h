@@ -14,6 +14,7 @@ struct CtxView {
     int device;
     uint32_t num_objects;
     uint32_t tick;              // last evaluated tick
+    uint32_t restores;          // snapshots restored so far (the tick may be the same after one, its log another)
     uint32_t min_meet;
     bool evaluated;
     const unsigned long long *keys;   // the tick's pairs (bit 63: a tag, masked off by readers)

@@ -4104,6 +4104,7 @@ struct glint_ctx {
     bool has_prev = false;
     uint32_t tick = 0;
     uint32_t prev_tick = 0;
+    uint32_t restores = 0;
     uint32_t scan_blocks = 0;
     uint32_t join_blocks = 1024;   // workgroups of the join
     uint32_t fused_join_blocks = 1024;   // its share of a fused join: about one per 1024 objects, 64 to 1024
@@ -4993,6 +4994,7 @@ glint_status glint_ctx_view(glint_ctx *c, CtxView *v)
     v->device = c->device;
     v->num_objects = c->s.n;
     v->tick = c->prev_tick;
+    v->restores = c->restores;
     v->min_meet = c->s.min_meet;
     v->evaluated = c->evaluated && c->has_prev;
     // after evaluate the current tick's pairs are the previous generation
@@ -5861,6 +5863,7 @@ glint_status glint_restore(glint_ctx *c, const void *buf, uint64_t bytes)
     }
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
+    c->restores++;
     c->cur_gen = (int)h.cur_gen;   // the sections follow the generation parity of the snapshot
     const uint8_t *p = static_cast<const uint8_t *>(buf) + sizeof h;
     const std::vector<Section> v = state_sections(c, h.gen_count, h.mlog_count, h.kvlog_count);

@@ -634,8 +634,9 @@ glint_status start_query(glint_server *s, Query &q, int slot)
     glint_ctx_view(s->ctx, &v);
     // the log as the server's last tick left it (asking the context would
     // wait for the queries before this one), unless ticks ran beside the server
+    // or a snapshot was restored under it
     uint64_t total = s->log_total, first = s->log_first;
-    if (v.tick != s->view.tick) {
+    if (v.tick != s->view.tick || v.restores != s->view.restores) {
         const glint_status gs = glint_meeting_log_info(s->ctx, &total, &first);
         if (gs) return gs;
     }
