@@ -59,11 +59,15 @@ constexpr int kBorderStage = 512;                   // staged border objects per
 enum JoinSum : uint32_t { kSumContacts, kSumBorder, kSumDup, kSumStored, kSumBand, kSumTests, kSumEvals, kJoinSums };
 constexpr uint32_t kJoinParts = 64;
 constexpr uint32_t kJoinPartStride = 16;            // 128 B
+// Words of the join's queues, a line each: leaves of the list dealt out (and,
+// above, whether leaves were handed over), and those handed over.
+constexpr uint32_t kQueueLeaves = 0, kQueueHanded = 16, kQueueWords = 32;
 // A tick with at least this many meetings has them sorted on the device for
 // the caller; below, the host sorts them as fast as the sort's launches take
 // (update_meetings with 512 meetings 84 us against 74 by the host, 1024: 89
 // and 93, 2048: 198 and 203, 8192: 241 and 470, 65536: 570 and 3170).
 constexpr uint64_t kOrderMeetings = 2048;
+constexpr uint32_t kMaxJoinBlocks = 1024;           // workgroups of a context's join at most
 constexpr uint32_t kHeavyLeaf = 256;                // leaves above this size are joined first
 constexpr uint32_t kSparseMax = 512;                // most objects of a leaf joined by one wave
 // and most objects per reach x reach square of it.  Denser leaves have
@@ -424,6 +428,7 @@ __device__ __forceinline__ void stamp_end(TickParams *tp)
 __device__ __forceinline__ void reset_tick_body(const DevState &s)
 {
     for (uint32_t k = threadIdx.x; k < kJoinParts * kJoinPartStride; k += blockDim.x) s.jpart[k] = 0;
+    if (threadIdx.x == 0) s.join_queue[kQueueLeaves] = s.join_queue[kQueueHanded] = 0;
     for (uint32_t k = threadIdx.x; k < s.coarse_max; k += blockDim.x) s.bins[k * kBinStride] = 0;
     if (threadIdx.x != 0) return;
     Counters *c = s.ctr;
@@ -449,7 +454,6 @@ __device__ __forceinline__ void reset_tick_body(const DevState &s)
     c->n_drop_objs = 0;
     c->n_tests = 0;
     c->n_evals = 0;
-    c->work_inside = 0;
     c->g_heavy = 0;
 }
 
@@ -2636,6 +2640,23 @@ struct JoinLds {
 // test, the key and its flags follow 64 pairs at a time, from the sorted
 // arrays: an object's ids and candidate lists are only read where a contact
 // needs them (the tiles read them for every object).
+// A leaf sparse on average may hold a crowd, or have a crowd's units aimed at
+// it.  A wave decides 64 pairs in about 1.3 us and tests a column of 64 rows in
+// about 80 ns, and holds up the launch alone, where the tiles have a workgroup
+// and all of it in LDS.  Such leaves are handed over to the tiles (hand_over):
+// with at most kSparseFew sparse leaves, when a crowd shows in the cells
+// (kSparseCell) or past kSparsePairsFew pairs or kSparseSteps columns; with
+// more, past kSparsePairs, since a wave per leaf then does more at once than a
+// workgroup per leaf.  A leaf's pairs are not decided before its end, so nothing
+// of it has to be taken back: those that the stage has no room for wait in
+// memory (SparseWave::past).  Ticks in us where the tiles join every leaf / no
+// leaf is handed over / as it is: 320 objects in one spot of a kilometre 320 /
+// 1230 / 311, 160 there 160 / 356 / 130, 40 there 106 / 75 / 76, 400 over 100 m of
+// two kilometres 132 / 267 / 102, 500 objects beside 12 of another leaf 590 / 3290
+// / 540, 120 in one spot among 100k uniform ones 305 / 258 / 142, 100k in spots of
+// 100 447 / 801 / 351, of 20 331 / 258 / 245 (at 1000 pairs 228, at 2000 267), of 5
+// 348 / 161 / 161, 1M in hotspots 1036 / 595 / 600; 256 leaves of 300 over 100 m
+// 194 / 157 / 119 (at 448 columns 180).
 // A leaf of 100 objects takes a wave about 5 us, nearly all of it waiting:
 // the leaf's record and positions (2 us), the sort (1.3), the runs (1.7).
 // The join of 1M uniform objects went from 297 to 39 us, of 300k in lon/lat
@@ -2643,7 +2664,14 @@ struct JoinLds {
 // from 3.2 to 0.5 ms.
 constexpr uint32_t kSparseSide = 16;
 constexpr uint32_t kSparseCells = kSparseSide * kSparseSide;
-constexpr uint32_t kSparseStage = 128;   // staged pairs, and stored keys, of a wave
+constexpr uint32_t kSparseStage = 368;   // staged pairs of a wave (what the tiles' LDS leaves room for)
+constexpr uint32_t kSparseOut = 128;     // keys of a wave
+constexpr uint32_t kSparseFew = 256;     // sparse leaves of a tick up to which each has a CU to itself
+constexpr uint32_t kSparseCell = 128;    // most objects of a cell then (96, 128 and 192 take the same)
+constexpr uint32_t kSparseSteps = 1024;  // and most columns
+constexpr uint32_t kSparsePairsFew = 600;   // and most pairs (40 objects in one spot, 780, take the same either way)
+constexpr uint32_t kSparsePairs = 1500;  // most pairs of a leaf with more leaves
+constexpr uint32_t kSparseCols = 8;      // columns a lane tests at once (1, 4, 8: 165, 105, 80 ns a column)
 constexpr int kSparsePer = (int)(kSparseMax / 64);
 
 // A workgroup's counts, in the order of JoinSum.
@@ -2658,12 +2686,14 @@ struct SparseLds {
     uint16_t at[kSparseMax];              // their place in the leaf's run of the sorted arrays
     uint32_t start[kSparseCells + 4];     // first object of every cell, and the count at the end
     uint2 stage[kSparseStage];            // staged pairs: row (sorted index, or unit), column (kSparseUnit: a unit row)
-    unsigned long long out[kSparseStage]; // keys of contacts to be stored
+    unsigned long long out[kSparseOut];   // keys of contacts to be stored
 };
 constexpr uint32_t kSparseUnit = 0x80000000u;
+constexpr uint32_t kHandedOver = 0xFFFFFFFEu;   // (node ids are below)
 
 // A wave's sums over its sparse leaves (per lane unless stated).
 struct SparseWave {
+    uint2 *past;                       // where the pairs of a leaf past the stage's end go
     uint32_t n, nout;                  // staged pairs and keys (uniform)
     uint32_t kept;                     // keys in all (uniform)
     uint32_t pass_in, pass_bd;         // contacts
@@ -2746,15 +2776,17 @@ __device__ __forceinline__ void sparse_drain(const DevState &s, const TickView &
     wave_sync();
     const uint32_t lane = lane_id(), m = min(w.n, 64u);
     w.n -= m;
+    const uint32_t i = w.n + lane;
     const unsigned long long key =
-        lane < m ? sparse_key<GEO>(s, tv, has_prev, w, L.stage[w.n + lane]) : kEmptyKey;
+        lane < m ? sparse_key<GEO>(s, tv, has_prev, w, i < kSparseStage ? L.stage[i] : w.past[i - kSparseStage])
+                 : kEmptyKey;
     const unsigned long long keep = __builtin_amdgcn_ballot_w64(key != kEmptyKey);
     if (key != kEmptyKey) L.out[w.nout + __popcll(keep & ((1ull << lane) - 1ull))] = key;
     const uint32_t cnt = (uint32_t)__popcll(keep);
     w.nout += cnt;
     w.kept += cnt;
     wave_sync();
-    if (w.nout > kSparseStage - 64) {
+    if (w.nout > kSparseOut - 64) {
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(&s.ctr->n_clist, (unsigned long long)w.nout);
         sparse_write(s, L.out, w.nout, __shfl(base, 0));
@@ -2763,11 +2795,21 @@ __device__ __forceinline__ void sparse_drain(const DevState &s, const TickView &
     }
 }
 
-template <bool GEO>
-__device__ __forceinline__ void join_sparse(const DevState &s, const TickView &tv, bool has_prev, SparseLds &L,
-                                            SparseWave &w, uint32_t leaf)
+// Column t of a row whose columns are three runs: those before n1, those
+// before n2 and the rest, each moved by its distance.
+__device__ __forceinline__ uint32_t sparse_column(uint32_t t, uint32_t n1, uint32_t n2, uint32_t d1, uint32_t d2,
+                                                  uint32_t d3)
 {
-    const uint32_t lane = lane_id();
+    return t + (t < n1 ? d1 : t < n2 ? d2 : d3);
+}
+
+// False for a leaf that is left to the tiles: none of its pairs is staged then.
+// few: at most kSparseFew leaves are sparse.
+template <bool GEO>
+__device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &tv, SparseLds &L,
+                                            SparseWave &w, uint32_t leaf, bool few)
+{
+    const uint32_t lane = lane_id(), before_leaf = w.n;
     const uint32_t off = s.offset[leaf], cnt = s.count[leaf];
     const uint32_t uoff = s.ustart[leaf], ucnt = s.ucount[leaf];
     const double2 lo = reinterpret_cast<const double2 *>(s.nodes + leaf)[1], hi = node_high(s.nodes, leaf);
@@ -2779,7 +2821,7 @@ __device__ __forceinline__ void join_sparse(const DevState &s, const TickView &t
         y[q] = k < cnt ? tv.sy[off + k] : 0.0;
     }
     // the first units' sorted positions, in flight meanwhile
-    uint32_t ug = lane < ucnt ? reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + lane)[3] : 0u;
+    const uint32_t ug = lane < ucnt ? reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + lane)[3] : 0u;
     wave_sync();
     reinterpret_cast<uint4 *>(L.start)[lane] = make_uint4(0u, 0u, 0u, 0u);
     const double2 r = sparse_reach(s, lo.y, hi.y);
@@ -2816,6 +2858,7 @@ __device__ __forceinline__ void join_sparse(const DevState &s, const TickView &t
     wave_sync();
     {
         const uint4 c = reinterpret_cast<uint4 *>(L.start)[lane];
+        if (few && __builtin_amdgcn_ballot_w64(max(max(c.x, c.y), max(c.z, c.w)) > kSparseCell)) return false;
         const uint32_t v = c.x + c.y + c.z + c.w;
         const uint32_t before = wave_inclusive_scan(v) - v;
         reinterpret_cast<uint4 *>(L.start)[lane] =
@@ -2832,65 +2875,123 @@ __device__ __forceinline__ void join_sparse(const DevState &s, const TickView &t
         }
     }
     wave_sync();
-    // The columns of a lane's row: up to three runs of the sorted order, one
-    // object per step and lane.
-    auto scan = [&](float2 row, uint32_t ex, uint32_t flag, uint32_t a0, uint32_t na, uint32_t b0, uint32_t nb,
-                    uint32_t c0, uint32_t nc) {
-        const uint32_t n = na + nb + nc;
-        const int dab = (int)b0 - (int)na, dbc = (int)c0 - (int)(na + nb);
-        for (uint32_t t = 0; __builtin_amdgcn_ballot_w64(t < n) != 0ull; t++) {
-            const bool live = t < n;
-            const uint32_t j = live ? (uint32_t)((int)t + (t < na ? (int)a0 : t < na + nb ? dab : dbc)) : 0u;
-            const float2 c = L.pos[j];
-            const float dx = row.x - c.x, dy = row.y - c.y;
-            const bool hit = live && dist2_f32(dx, dy) <= lim;
-            const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
-            w.evals++;
-            if (!m) continue;
-            if (hit) L.stage[w.n + __popcll(m & ((1ull << lane) - 1ull))] = make_uint2(ex, (off + L.at[j]) | flag);
-            w.n += (uint32_t)__popcll(m);
-            if (w.n > kSparseStage - 64) sparse_drain<GEO>(s, tv, has_prev, L, w);
-        }
-    };
-    // run of the cells beside c (and its own) in the row of cells dy above
-    auto run_of = [&](uint2 c, int dy, uint32_t &b, uint32_t &n) {
+    // run of the cells beside c (and its own) in the row of cells dy above:
+    // its first object and their number
+    auto run_of = [&](uint2 c, int dy) {
         const int cy = (int)c.y + dy;
-        b = 0;
-        n = 0;
-        if (cy < 0 || cy >= (int)kSparseSide) return;
+        if (cy < 0 || cy >= (int)kSparseSide) return make_uint2(0u, 0u);
         const uint32_t base = (uint32_t)cy * kSparseSide;
-        b = L.start[base + (c.x ? c.x - 1 : 0u)];
-        n = L.start[base + min(c.x + 2, kSparseSide)] - b;
+        const uint32_t first = L.start[base + (c.x ? c.x - 1 : 0u)];
+        return make_uint2(first, L.start[base + min(c.x + 2, kSparseSide)] - first);
     };
-    for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
-        const uint32_t i = i0 + lane;
-        const bool vi = i < cnt;
-        const float2 row = vi ? L.pos[i] : make_float2(0.0f, 0.0f);
-        uint32_t b0 = 0, nb = 0, c0 = 0, nc = 0, g = 0;
-        if (vi) {
-            const uint2 c = cell_of(row);
-            g = off + L.at[i];
-            run_of(c, 0, b0, nb);
-            nb = b0 + nb - (i + 1);   // the rest of the run
-            run_of(c, 1, c0, nc);
+    // 64 rows at a time: a lane's columns are up to three runs of the sorted
+    // order.  False past the wave's bounds.
+    const uint32_t most = before_leaf + (few ? kSparsePairsFew : kSparsePairs);
+    const unsigned long long most_evals = w.evals + kSparseSteps;
+    auto scan = [&](float2 row, uint32_t ex, uint32_t flag, uint2 below, uint2 own, uint2 above) -> bool {
+        const uint32_t n1 = below.y, n2 = n1 + own.y, n = n2 + above.y;
+        const uint32_t d1 = below.x, d2 = own.x - n1, d3 = above.x - n2;
+        for (uint32_t t = 0; __builtin_amdgcn_ballot_w64(t < n) != 0ull; t += kSparseCols) {
+            float2 c[kSparseCols];
+#pragma unroll
+            for (uint32_t q = 0; q < kSparseCols; q++)
+                c[q] = L.pos[t + q < n ? sparse_column(t + q, n1, n2, d1, d2, d3) : 0u];
+            uint32_t hits = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < kSparseCols; q++)
+                hits |= t + q < n && dist2_f32(row.x - c[q].x, row.y - c[q].y) <= lim ? 1u << q : 0u;
+            w.evals += kSparseCols;
+            for (unsigned long long m; (m = __builtin_amdgcn_ballot_w64(hits != 0u)) != 0ull; hits &= hits - 1) {
+                if (hits) {
+                    const uint32_t place = w.n + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                    const uint32_t j = sparse_column(t + __builtin_ctz(hits), n1, n2, d1, d2, d3);
+                    const uint2 e = make_uint2(ex, (off + L.at[j]) | flag);
+                    if (place < kSparseStage)
+                        L.stage[place] = e;
+                    else
+                        w.past[place - kSparseStage] = e;
+                }
+                w.n += (uint32_t)__popcll(m);
+                if (w.n > most) return false;
+            }
         }
-        scan(row, g, 0u, i + 1, nb, c0, nc, 0u, 0u);
-    }
-    for (uint32_t u0 = 0; u0 < ucnt; u0 += 64) {
-        const uint32_t u = u0 + lane;
-        float2 row = make_float2(0.0f, 0.0f);
-        uint32_t a0 = 0, na = 0, b0 = 0, nb = 0, c0 = 0, nc = 0;
-        if (u < ucnt) {
-            if (u0) ug = reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + u)[3];
-            row = make_float2((float)((tv.sx[ug] - lo.x) * ix), (float)((tv.sy[ug] - lo.y) * iy));
-            const uint2 c = cell_of(row);
-            run_of(c, -1, a0, na);
-            run_of(c, 0, b0, nb);
-            run_of(c, 1, c0, nc);
+        return !few || w.evals <= most_evals;
+    };
+    auto scan_leaf = [&]() -> bool {
+        for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
+            const uint32_t i = i0 + lane;
+            float2 row = make_float2(0.0f, 0.0f);
+            uint32_t g = 0;
+            uint2 own = make_uint2(0u, 0u), above = own;
+            if (i < cnt) {
+                row = L.pos[i];
+                const uint2 c = cell_of(row);
+                g = off + L.at[i];
+                own = run_of(c, 0);
+                own = make_uint2(i + 1, own.x + own.y - (i + 1));   // the rest of the run
+                above = run_of(c, 1);
+            }
+            if (!scan(row, g, 0u, make_uint2(0u, 0u), own, above)) return false;
         }
-        scan(row, uoff + u, kSparseUnit, a0, na, b0, nb, c0, nc);
+        for (uint32_t u0 = 0; u0 < ucnt; u0 += 64) {
+            const uint32_t u = u0 + lane;
+            float2 row = make_float2(0.0f, 0.0f);
+            uint2 below = make_uint2(0u, 0u), own = below, above = below;
+            if (u < ucnt) {
+                const uint32_t g = u0 ? reinterpret_cast<const uint32_t *>(s.unit_lf + uoff + u)[3] : ug;
+                row = make_float2((float)((tv.sx[g] - lo.x) * ix), (float)((tv.sy[g] - lo.y) * iy));
+                const uint2 c = cell_of(row);
+                below = run_of(c, -1);
+                own = run_of(c, 0);
+                above = run_of(c, 1);
+            }
+            if (!scan(row, uoff + u, kSparseUnit, below, own, above)) return false;
+        }
+        return true;
+    };
+    if (!scan_leaf()) {
+        w.n = before_leaf;
+        return false;
     }
+    if (w.n > kSparseStage) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // (w.past is read by other lanes)
     if (lane == 0) w.tests += (unsigned long long)cnt * (cnt - 1) / 2 + (unsigned long long)cnt * ucnt;
+    return true;
+}
+
+// The leaves handed over, a queue of the launch: a word with the numbers of
+// places listed (high) and taken (low), and the list.  Any workgroup takes them
+// when the leaf list is done, at the latest the one that listed a leaf, since it
+// goes on until every place is taken.  A workgroup that finds none leaves; a
+// place taken before it was listed has no taker left, and is passed over.
+// Whether there are any is told by the word that deals out the leaf list (its
+// high half): a look at the queue by every workgroup that is done had made the
+// join of 32 cities 5 to 10 % longer.
+__device__ __forceinline__ void hand_over(const DevState &s, uint32_t leaf)
+{
+    unsigned long long q;
+    do
+        q = atomicAdd(s.join_queue + kQueueHanded, 1ull << 32);
+    while ((uint32_t)q > (uint32_t)(q >> 32));   // (at most once per workgroup that left)
+    __hip_atomic_store(s.handed_list + (uint32_t)(q >> 32), leaf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    atomicAdd(s.join_queue + kQueueLeaves, 1ull << 32);
+}
+
+// The next of them, or kNone.  A place listed a moment ago may not be written
+// yet: its writer stores it right after it listed it, waiting for nothing.
+// The place is empty (kNone) again for the next tick.
+__device__ __forceinline__ uint32_t take_handed(const DevState &s)
+{
+    unsigned long long *queue = s.join_queue + kQueueHanded;
+    unsigned long long q = __hip_atomic_load(queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((uint32_t)q >= (uint32_t)(q >> 32)) return kNone;
+    q = atomicAdd(queue, 1ull);
+    if ((uint32_t)q >= (uint32_t)(q >> 32)) return kNone;
+    uint32_t leaf;
+    do
+        leaf = __hip_atomic_load(s.handed_list + (uint32_t)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (leaf == kNone);
+    __hip_atomic_store(s.handed_list + (uint32_t)q, kNone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return leaf;
 }
 
 // Upper-triangle task t of n row blocks -> (r <= q), row-major.
@@ -3091,12 +3192,10 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
         dups += jc.dup;
     };
 
-    // thread 0: takes the next leaf from the queue and leaves it in LDS
-    auto fetch_leaf = [&]() {
-        const uint32_t w = atomicAdd(&s.ctr->work_inside, 1u);
-        lds.item = w;
-        if (w < nl) {
-            const uint32_t leaf = s.leaf_list[w < nh ? s.node_cap - 1 - w : w - nh];
+    // thread 0: leaves a leaf (kNone: none) and its record in LDS
+    auto set_leaf = [&](uint32_t leaf) {
+        lds.item = leaf;
+        if (leaf < kHandedOver) {
             JoinLeaf L;
             L.off = s.offset[leaf];
             L.cnt = s.count[leaf];
@@ -3113,16 +3212,33 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
             lds.leaf = L;
         }
     };
+    // thread 0: takes the next leaf of the list; after its end, kHandedOver if leaves were handed over
+    auto fetch_leaf = [&]() {
+        const unsigned long long q = atomicAdd(s.join_queue + kQueueLeaves, 1ull);
+        const uint32_t w = (uint32_t)q;
+        set_leaf(w < nl ? s.leaf_list[w < nh ? s.node_cap - 1 - w : w - nh] : q >> 32 ? kHandedOver : kNone);
+    };
     // The sparse leaves first, one wave each: the queue of tiles after them
     // evens out what their shares differ by.  The keys that the waves still
     // hold at the end go out with one reservation.
     const uint32_t nsp = (s.ctr->error & kErrUnitCap) ? 0 : s.ctr->n_sparse;
-    if (blk.id() * (kBlock / 64) < nsp) {
+    const bool few = nsp <= kSparseFew;
+    const uint32_t waves = few ? 1u : kBlock / 64;   // of a workgroup that take leaves
+    if (blk.id() * waves < nsp) {
         SparseLds &L = shared.sparse[wave];
         SparseWave w{};
-        for (uint32_t k = blk.id() * (kBlock / 64) + wave; k < nsp; k += blk.count() * (kBlock / 64))
-            join_sparse<GEO>(s, tv, has_prev, L, w, __builtin_amdgcn_readfirstlane(s.sparse_list[k]));
-        while (w.n) sparse_drain<GEO>(s, tv, has_prev, L, w);
+        // (room that pass 1 of the bucketing uses after the join: kChunk entries a wave)
+        static_assert(kSparsePairs + 128 <= kChunk && sizeof(uint2) == sizeof(*s.clist2), "a leaf's pairs fit a share");
+        w.past = reinterpret_cast<uint2 *>(s.clist2) + (size_t)(blk.id() * (kBlock / 64) + wave) * kChunk;
+        for (uint32_t k = wave < waves ? blk.id() * waves + wave : nsp;; k += blk.count() * waves) {
+            const bool more = k < nsp;
+            if (more) {
+                const uint32_t leaf = __builtin_amdgcn_readfirstlane(s.sparse_list[k]);
+                if (!join_sparse<GEO>(s, tv, L, w, leaf, few) && lane == 0) hand_over(s, leaf);
+            }
+            while (w.n > (more ? 64u : 0u)) sparse_drain<GEO>(s, tv, has_prev, L, w);
+            if (!more) break;
+        }
         if (lane == 0) sums.left[wave] = w.nout;
         __syncthreads();
         uint32_t before = 0, all = 0;
@@ -3153,7 +3269,12 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
         const uint32_t item = lds.item;
         const JoinLeaf F = lds.leaf;
         __syncthreads();   // read by every thread before thread 0 takes the next leaf
-        if (item >= nl) break;
+        if (item == kNone) break;
+        if (item == kHandedOver) {
+            if (threadIdx.x == 0) set_leaf(take_handed(s));
+            __syncthreads();
+            continue;
+        }
         // The next leaf is taken once this one's first tile is loaded: thread
         // 0 waits on the queue and the leaf's record while the other waves
         // start on the tasks (read after the last barrier of this leaf).
@@ -4106,7 +4227,7 @@ struct glint_ctx {
     uint32_t prev_tick = 0;
     uint32_t restores = 0;
     uint32_t scan_blocks = 0;
-    uint32_t join_blocks = 1024;   // workgroups of the join
+    uint32_t join_blocks = kMaxJoinBlocks;   // workgroups of the join
     uint32_t fused_join_blocks = 1024;   // its share of a fused join: about one per 1024 objects, 64 to 1024
     uint32_t table_grid = 4096;    // workgroups of the table update (persistent over the regions)
     uint32_t fine_grid = 1024;     // workgroups of the fine bucketing pass (persistent over the bins)
@@ -4802,6 +4923,10 @@ glint_status glint_create(const glint_config *cfg, glint_ctx **out)
     ALLOC(s.merge_list, node_cap);
     ALLOC(s.leaf_list, node_cap);
     ALLOC(s.sparse_list, node_cap);
+    ALLOC(s.handed_list, node_cap + kMaxJoinBlocks);   // (every leaf once, and the places passed over)
+    ALLOC(s.join_queue, kQueueWords);
+    k_fill_u32<<<grid_for(node_cap + kMaxJoinBlocks), kBlock, 0, c->stream>>>(s.handed_list, kNone,
+                                                                              node_cap + kMaxJoinBlocks);
     ALLOC(s.sleafb[0], N);
     ALLOC(s.sleafb[1], N);
     ALLOC(s.parent, node_cap);

@@ -217,6 +217,8 @@ struct DevState {
     uint32_t *merge_list;
     uint32_t *leaf_list;
     uint32_t *sparse_list;  // leaves the join gives to one wave each
+    uint32_t *handed_list;  // those of them that the tiles join after all (kNone: no entry)
+    unsigned long long *join_queue;     // the join's queue words (kQueueLeaves, kQueueHanded)
     uint32_t *parent;       // per node: its parent (kNone for the root), for descents that start at the last leaf
     double4 *region;        // per node: the points the descent sends into it, (x.lo, x.hi] x (y.lo, y.hi]
     uint32_t incremental;   // objects are placed from their leaf of the tick before (not with the grid rebuild)
