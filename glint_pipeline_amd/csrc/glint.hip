@@ -24,6 +24,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "glint.h"
@@ -2642,7 +2643,7 @@ struct JoinLds {
 // needs them (the tiles read them for every object).
 // A leaf sparse on average may hold a crowd, or have a crowd's units aimed at
 // it.  A wave decides 64 pairs in about 1.3 us and tests a column of 64 rows in
-// about 80 ns, and holds up the launch alone, where the tiles have a workgroup
+// about 100 ns, and holds up the launch alone, where the tiles have a workgroup
 // and all of it in LDS.  Such leaves are handed over to the tiles (hand_over):
 // with at most kSparseFew sparse leaves, when a crowd shows in the cells
 // (kSparseCell) or past kSparsePairsFew pairs or kSparseSteps columns; with
@@ -2671,7 +2672,10 @@ constexpr uint32_t kSparseCell = 128;    // most objects of a cell then (96, 128
 constexpr uint32_t kSparseSteps = 1024;  // and most columns
 constexpr uint32_t kSparsePairsFew = 600;   // and most pairs (40 objects in one spot, 780, take the same either way)
 constexpr uint32_t kSparsePairs = 1500;  // most pairs of a leaf with more leaves
-constexpr uint32_t kSparseCols = 8;      // columns a lane tests at once (1, 4, 8: 165, 105, 80 ns a column)
+// Columns a lane tests at once.  1 / 4 / 8: a column takes 165 / 105 / 80 ns, but
+// most rows have a few (leaves of 40 uniform objects, 1.8M of them: join 93 / 87 /
+// 93 us), and the ones past a row's end are tested against a point beyond reach.
+constexpr uint32_t kSparseCols = 4;
 constexpr int kSparsePer = (int)(kSparseMax / 64);
 
 // A workgroup's counts, in the order of JoinSum.
@@ -2682,7 +2686,8 @@ struct JoinSums {
 };
 
 struct SparseLds {
-    float2 pos[kSparseMax];               // offsets from the leaf's low corner in reaches, cell order
+    float2 pos[kSparseMax + 1];           // offsets from the leaf's low corner in reaches, cell order, and one beyond reach
+    float2 pad;                           // (start is read 16 bytes at a time)
     uint16_t at[kSparseMax];              // their place in the leaf's run of the sorted arrays
     uint32_t start[kSparseCells + 4];     // first object of every cell, and the count at the end
     uint2 stage[kSparseStage];            // staged pairs: row (sorted index, or unit), column (kSparseUnit: a unit row)
@@ -2795,14 +2800,6 @@ __device__ __forceinline__ void sparse_drain(const DevState &s, const TickView &
     }
 }
 
-// Column t of a row whose columns are three runs: those before n1, those
-// before n2 and the rest, each moved by its distance.
-__device__ __forceinline__ uint32_t sparse_column(uint32_t t, uint32_t n1, uint32_t n2, uint32_t d1, uint32_t d2,
-                                                  uint32_t d3)
-{
-    return t + (t < n1 ? d1 : t < n2 ? d2 : d3);
-}
-
 // False for a leaf that is left to the tiles: none of its pairs is staged then.
 // few: at most kSparseFew leaves are sparse.
 template <bool GEO>
@@ -2888,32 +2885,41 @@ __device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &t
     // order.  False past the wave's bounds.
     const uint32_t most = before_leaf + (few ? kSparsePairsFew : kSparsePairs);
     const unsigned long long most_evals = w.evals + kSparseSteps;
-    auto scan = [&](float2 row, uint32_t ex, uint32_t flag, uint2 below, uint2 own, uint2 above) -> bool {
-        const uint32_t n1 = below.y, n2 = n1 + own.y, n = n2 + above.y;
+    auto scan = [&](auto unit, float2 row, uint32_t ex, uint2 below, uint2 own, uint2 above) -> bool {
+        constexpr uint32_t flag = decltype(unit)::value ? kSparseUnit : 0u;   // (an object has no run below)
+        const uint32_t n1 = flag ? below.y : 0u, n2 = n1 + own.y, n = n2 + above.y;
         const uint32_t d1 = below.x, d2 = own.x - n1, d3 = above.x - n2;
         for (uint32_t t = 0; __builtin_amdgcn_ballot_w64(t < n) != 0ull; t += kSparseCols) {
             float2 c[kSparseCols];
+            uint32_t j[kSparseCols];
+            unsigned long long m[kSparseCols], any = 0;
 #pragma unroll
-            for (uint32_t q = 0; q < kSparseCols; q++)
-                c[q] = L.pos[t + q < n ? sparse_column(t + q, n1, n2, d1, d2, d3) : 0u];
-            uint32_t hits = 0;
+            for (uint32_t q = 0; q < kSparseCols; q++) {
+                j[q] = t + q < n ? t + q + (flag && t + q < n1 ? d1 : t + q < n2 ? d2 : d3) : kSparseMax;
+                c[q] = L.pos[j[q]];
+            }
 #pragma unroll
-            for (uint32_t q = 0; q < kSparseCols; q++)
-                hits |= t + q < n && dist2_f32(row.x - c[q].x, row.y - c[q].y) <= lim ? 1u << q : 0u;
+            for (uint32_t q = 0; q < kSparseCols; q++) {
+                m[q] = __builtin_amdgcn_ballot_w64(dist2_f32(row.x - c[q].x, row.y - c[q].y) <= lim);
+                any |= m[q];
+            }
             w.evals += kSparseCols;
-            for (unsigned long long m; (m = __builtin_amdgcn_ballot_w64(hits != 0u)) != 0ull; hits &= hits - 1) {
-                if (hits) {
-                    const uint32_t place = w.n + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                    const uint32_t j = sparse_column(t + __builtin_ctz(hits), n1, n2, d1, d2, d3);
-                    const uint2 e = make_uint2(ex, (off + L.at[j]) | flag);
+            if (!any) continue;
+#pragma unroll
+            for (uint32_t q = 0; q < kSparseCols; q++) {
+                if (!m[q]) continue;
+                if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
+                    const uint32_t place = w.n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m[q] >> 32),
+                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m[q], 0u));
+                    const uint2 e = make_uint2(ex, (off + L.at[j[q]]) | flag);
                     if (place < kSparseStage)
                         L.stage[place] = e;
                     else
                         w.past[place - kSparseStage] = e;
                 }
-                w.n += (uint32_t)__popcll(m);
-                if (w.n > most) return false;
+                w.n += (uint32_t)__popcll(m[q]);
             }
+            if (w.n > most) return false;
         }
         return !few || w.evals <= most_evals;
     };
@@ -2931,7 +2937,7 @@ __device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &t
                 own = make_uint2(i + 1, own.x + own.y - (i + 1));   // the rest of the run
                 above = run_of(c, 1);
             }
-            if (!scan(row, g, 0u, make_uint2(0u, 0u), own, above)) return false;
+            if (!scan(std::false_type{}, row, g, make_uint2(0u, 0u), own, above)) return false;
         }
         for (uint32_t u0 = 0; u0 < ucnt; u0 += 64) {
             const uint32_t u = u0 + lane;
@@ -2945,7 +2951,7 @@ __device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &t
                 own = run_of(c, 0);
                 above = run_of(c, 1);
             }
-            if (!scan(row, uoff + u, kSparseUnit, below, own, above)) return false;
+            if (!scan(std::true_type{}, row, uoff + u, below, own, above)) return false;
         }
         return true;
     };
@@ -3223,12 +3229,15 @@ __device__ __forceinline__ void join_body(const DevState s, const P blk)
     // hold at the end go out with one reservation.
     const uint32_t nsp = (s.ctr->error & kErrUnitCap) ? 0 : s.ctr->n_sparse;
     const bool few = nsp <= kSparseFew;
-    const uint32_t waves = few ? 1u : kBlock / 64;   // of a workgroup that take leaves
+    // (its first wave only while a quarter of the workgroups takes them all)
+    const uint32_t waves = nsp * (kBlock / 64) <= blk.count() ? 1u : kBlock / 64;
     if (blk.id() * waves < nsp) {
         SparseLds &L = shared.sparse[wave];
         SparseWave w{};
         // (room that pass 1 of the bucketing uses after the join: kChunk entries a wave)
-        static_assert(kSparsePairs + 128 <= kChunk && sizeof(uint2) == sizeof(*s.clist2), "a leaf's pairs fit a share");
+        static_assert(kSparsePairs + 64 * (kSparseCols + 1) <= kChunk && sizeof(uint2) == sizeof(*s.clist2),
+                      "a leaf's pairs fit a share");
+        if (lane == 0) L.pos[kSparseMax] = make_float2(__builtin_inff(), __builtin_inff());
         w.past = reinterpret_cast<uint2 *>(s.clist2) + (size_t)(blk.id() * (kBlock / 64) + wave) * kChunk;
         for (uint32_t k = wave < waves ? blk.id() * waves + wave : nsp;; k += blk.count() * waves) {
             const bool more = k < nsp;
