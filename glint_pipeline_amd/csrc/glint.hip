@@ -62,7 +62,9 @@ constexpr uint32_t kJoinParts = 64;
 constexpr uint32_t kJoinPartStride = 16;            // 128 B
 // Words of the join's queues, a line each: leaves of the list dealt out (and,
 // above, whether leaves were handed over), and those handed over.
-constexpr uint32_t kQueueLeaves = 0, kQueueHanded = 16, kQueueWords = 32;
+constexpr uint32_t kQueueLeaves = 0, kQueueHanded = 16;
+// and the workgroups of the schema update that are done.
+constexpr uint32_t kQueueSchema = 32, kQueueWords = 48;
 // A tick with at least this many meetings has them sorted on the device for
 // the caller; below, the host sorts them as fast as the sort's launches take
 // (update_meetings with 512 meetings 84 us against 74 by the host, 1024: 89
@@ -429,7 +431,7 @@ __device__ __forceinline__ void stamp_end(TickParams *tp)
 __device__ __forceinline__ void reset_tick_body(const DevState &s)
 {
     for (uint32_t k = threadIdx.x; k < kJoinParts * kJoinPartStride; k += blockDim.x) s.jpart[k] = 0;
-    if (threadIdx.x == 0) s.join_queue[kQueueLeaves] = s.join_queue[kQueueHanded] = 0;
+    if (threadIdx.x < kQueueWords) s.join_queue[threadIdx.x] = 0;
     for (uint32_t k = threadIdx.x; k < s.coarse_max; k += blockDim.x) s.bins[k * kBinStride] = 0;
     if (threadIdx.x != 0) return;
     Counters *c = s.ctr;
@@ -584,87 +586,83 @@ __global__ void k_build_collect(DevState s)
     }
 }
 
-// Split the listed leaves one level.  build_boxes selects the child boxes of
-// the initial build, (lo, mid) and (mid, hi) (QTree.h:163-166); otherwise the
-// elastic update's lo + half and mid + half (geometry.cu:1151-1156).
-template <class P>
-__device__ __forceinline__ void split_body(const DevState s, const P blk, int build_boxes)
+// Splits a leaf one level; its children are the four entries below `top` of
+// the free stack.  build_boxes selects the child boxes of the initial build,
+// (lo, mid) and (mid, hi) (QTree.h:163-166); otherwise the elastic update's
+// lo + half and mid + half (geometry.cu:1151-1156).
+__device__ __forceinline__ void split_node(const DevState &s, uint32_t node, int32_t top, int build_boxes)
 {
-    uint32_t ns = s.ctr->n_split;
-    for (uint32_t k = blk.id() * blockDim.x + threadIdx.x; k < ns; k += blk.count() * blockDim.x) {
-        uint32_t node = s.split_list[k];
-        int32_t top = atomicSub(&s.ctr->free_top, 4);
+    Node p = s.nodes[node];
+    NodeMeta pm = s.meta[node];
+    double xhalf = p.mx - p.lx;
+    double yhalf = p.my - p.ly;
+    Node np = p;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t c = (uint32_t)s.free_stack[top - 1 - i];
+        Node ch;
+        if (build_boxes) {
+            ch.lx = (i & 1) ? p.mx : p.lx;
+            ch.hx = (i & 1) ? p.hx : p.mx;
+            ch.ly = (i & 2) ? p.my : p.ly;
+            ch.hy = (i & 2) ? p.hy : p.my;
+        } else {
+            ch.lx = p.lx + (double)(i % 2 == 1) * xhalf;
+            ch.ly = p.ly + (double)(i / 2 == 1) * yhalf;
+            ch.hx = p.mx + (double)(i % 2 == 1) * xhalf;
+            ch.hy = p.my + (double)(i / 2 == 1) * yhalf;
+        }
+        ch.mx = (ch.lx + ch.hx) / 2;
+        ch.my = (ch.ly + ch.hy) / 2;
+        ch.child[0] = kLeafTag;
+        ch.child[1] = ch.child[2] = ch.child[3] = 0;
+        s.nodes[c] = ch;
+        s.parent[c] = node;
+        NodeMeta m;
+        m.type = kLeaf;
+        m.level = pm.level + 1;
+        m.overflow = 0;
+        m.underflow = 0;
+        s.meta[c] = m;
+        np.child[i] = c;
+    }
+    s.nodes[node] = np;
+    pm.type = kBranch;
+    s.meta[node] = pm;
+}
+
+// The listed leaves of the initial build.
+__global__ void k_split(DevState s)
+{
+    const uint32_t ns = s.ctr->n_split;
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < ns; k += gridDim.x * blockDim.x) {
+        const int32_t top = atomicSub(&s.ctr->free_top, 4);
         if (top < 4) {
             atomicAdd(&s.ctr->free_top, 4);   // give the entries back: the pool never goes negative
             atomicOr(&s.ctr->error, kErrNodeCap);
             continue;
         }
-        Node p = s.nodes[node];
-        NodeMeta pm = s.meta[node];
-        double xhalf = p.mx - p.lx;
-        double yhalf = p.my - p.ly;
-        Node np = p;
-        for (int i = 0; i < 4; i++) {
-            uint32_t c = (uint32_t)s.free_stack[top - 1 - i];
-            Node ch;
-            if (build_boxes) {
-                ch.lx = (i & 1) ? p.mx : p.lx;
-                ch.hx = (i & 1) ? p.hx : p.mx;
-                ch.ly = (i & 2) ? p.my : p.ly;
-                ch.hy = (i & 2) ? p.hy : p.my;
-            } else {
-                ch.lx = p.lx + (double)(i % 2 == 1) * xhalf;
-                ch.ly = p.ly + (double)(i / 2 == 1) * yhalf;
-                ch.hx = p.mx + (double)(i % 2 == 1) * xhalf;
-                ch.hy = p.my + (double)(i / 2 == 1) * yhalf;
-            }
-            ch.mx = (ch.lx + ch.hx) / 2;
-            ch.my = (ch.ly + ch.hy) / 2;
-            ch.child[0] = kLeafTag;
-            ch.child[1] = ch.child[2] = ch.child[3] = 0;
-            s.nodes[c] = ch;
-            s.parent[c] = node;
-            NodeMeta m;
-            m.type = kLeaf;
-            m.level = pm.level + 1;
-            m.overflow = 0;
-            m.underflow = 0;
-            s.meta[c] = m;
-            np.child[i] = c;
-        }
-        s.nodes[node] = np;
-        pm.type = kBranch;
-        s.meta[node] = pm;
+        split_node(s, s.split_list[k], top, 1);
     }
 }
 
-__global__ void k_split(DevState s) { split_body(s, this_blk(), 1); }   // (the initial build)
-// geometry.cu:1166-1190: the four leaf children return to the pool.
-template <class P>
-__device__ __forceinline__ void merge_body(const DevState s, const P blk)
+// geometry.cu:1166-1190: the four leaf children return to the pool (`freed`:
+// their places).
+__device__ __forceinline__ void merge_node(const DevState &s, uint32_t node, uint32_t *freed)
 {
-    uint32_t nm = s.ctr->n_merge;
-    for (uint32_t k = blk.id() * blockDim.x + threadIdx.x; k < nm; k += blk.count() * blockDim.x) {
-        uint32_t node = s.merge_list[k];
-        Node p = s.nodes[node];
-        int32_t top = atomicAdd(&s.ctr->free_top, 4);
-        if (top < 0 || top + 4 > (int32_t)s.node_cap) {
-            atomicOr(&s.ctr->error, kErrNodeCap);
-            continue;
-        }
-        for (int i = 0; i < 4; i++) {
-            uint32_t c = p.child[i];
-            s.meta[c].type = kInvalid;
-            s.free_stack[top + i] = (int32_t)c;
-        }
-        p.child[0] = kLeafTag;
-        p.child[1] = p.child[2] = p.child[3] = 0;
-        s.nodes[node] = p;
-        NodeMeta pm = s.meta[node];
-        pm.type = kLeaf;
-        pm.overflow = 0;
-        s.meta[node] = pm;
+    const uint4 ch = node_children(s.nodes, node);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t c = pick_child(ch, i);
+        s.meta[c].type = kInvalid;
+        freed[i] = c;
     }
+    s.nodes[node].child[0] = kLeafTag;
+    s.nodes[node].child[1] = s.nodes[node].child[2] = s.nodes[node].child[3] = 0;
+    NodeMeta pm = s.meta[node];
+    pm.type = kLeaf;
+    pm.overflow = 0;
+    s.meta[node] = pm;
 }
 
 // geometry.cu:1193-1234: decisions from this tick's counts, before any
@@ -754,25 +752,70 @@ __device__ __forceinline__ void schema_done(const DevState &s)
     if (s.mlog) c->n_mlog += c->n_meet < s.meet_cap ? c->n_meet : s.meet_cap;
 }
 
-// End of a tick, one workgroup: the listed leaves split, the listed branches
-// merged, the totals advanced and, in a run, the tick stamped.  A tick
-// changes few leaves (about 800 of 80k at 10M objects in hotspots), so the
-// four launches that did this had been waiting, 4.5 us each.
+// End of a tick: the listed leaves split, the listed branches merged, the
+// totals advanced and, in a run, the tick stamped.  A tick changes few leaves
+// (about 800 of 80k at 10M objects in hotspots), which the first workgroup does
+// alone: the four launches that did this had been waiting, 4.5 us each.  Where
+// more than kSchemaAlone leaves split or merge, all workgroups share them, since
+// one is slow with many.  One workgroup / 32 (with the four launches): 32 of
+// each 8 us / - (27), 512 16 / 21 (32), 2048 34 / 23 (33), 8192 210 / 34 (41),
+// 32768 940 / 89 (75); 64 workgroups took 28 for 512 and 41 for 8192.
+// Split k takes the k-th four entries from the top of the free stack.  The
+// entries that merges give back lie where splits may still be reading, so they
+// go there after every split: after a barrier of the one workgroup, or by the
+// last of several (from behind the merge list: a merge's five nodes are no
+// others', so there is room).
 constexpr int kSchemaThreads = 1024;
-__device__ __forceinline__ void schema_body(const DevState &s, bool run)
+constexpr uint32_t kSchemaAlone = 512;
+constexpr uint32_t kSchemaBlocks = 32;        // workgroups of a context alone
+constexpr uint32_t kSchemaBlocksFused = 8;    // and of a member of a fused group
+__device__ __forceinline__ void schema_body(const DevState &s, const Blk blk, bool run)
 {
-    if (threadIdx.x == kSchemaThreads - 1) schema_done(s);   // (beside the splits: it reads counts they leave alone)
-    split_body(s, Blk{0, 1}, 0);
+    const uint32_t ns = s.ctr->n_split, nm = s.ctr->n_merge;
+    const bool alone = max(ns, nm) <= kSchemaAlone;
+    if (blk.id() != 0 && alone) return;
+    const int32_t top = s.ctr->free_top;   // (changed at the end)
+    if (blk.id() == 0 && threadIdx.x == kSchemaThreads - 1) schema_done(s);   // (it reads counts that stay)
+    const uint32_t nblk = alone ? 1u : blk.count(), first = (threadIdx.x / 64 * nblk + blk.id()) * 64 + lane_id();
+    for (uint32_t k = first; k < ns; k += kSchemaThreads * nblk) {
+        if (top - 4 * (int64_t)k < 4)
+            atomicOr(&s.ctr->error, kErrNodeCap);
+        else
+            split_node(s, s.split_list[k], top - 4 * (int32_t)k, 0);
+    }
+    const uint32_t left = max(top, 0) - 4 * min(ns, (uint32_t)max(top, 0) / 4);   // entries the splits leave
+    uint32_t *back = reinterpret_cast<uint32_t *>(s.free_stack) + left;
+    uint32_t *freed = alone ? back : s.merge_list + nm;
+    if (max(left, nm) + 4ull * nm > s.node_cap) {   // (more nodes given back than there are)
+        if (threadIdx.x == 0) atomicOr(&s.ctr->error, kErrNodeCap);
+        return;
+    }
     __syncthreads();
-    merge_body(s, Blk{0, 1});
+    for (uint32_t k = first; k < nm; k += kSchemaThreads * nblk) merge_node(s, s.merge_list[k], freed + 4 * (size_t)k);
+    if (!alone) {
+        __shared__ bool last;
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) last = atomicAdd(s.join_queue + kQueueSchema, 1ull) + 1 == nblk;
+        __syncthreads();
+        if (!last) return;
+        __threadfence();
+        for (uint32_t k = threadIdx.x; k < 4 * nm; k += kSchemaThreads) back[k] = freed[k];
+        if (threadIdx.x == 0) s.join_queue[kQueueSchema] = 0;
+    }
     __syncthreads();
+    if (threadIdx.x == 0) s.ctr->free_top = (int32_t)(left + 4 * nm);
     if (run && threadIdx.x == 0) stamp_end(s.tp);
 }
 
-__global__ __launch_bounds__(kSchemaThreads) void k_schema(DevState s, bool run) { schema_body(s, run); }
+__global__ __launch_bounds__(kSchemaThreads) void k_schema(DevState s, bool run)
+{
+    schema_body(s, Blk{blockIdx.x, gridDim.x}, run);
+}
 __global__ __launch_bounds__(kSchemaThreads) void kf_schema(const Many m, bool run)
 {
-    schema_body(m.ss[member_of(m).i], run);
+    const Member w = member_of(m);
+    schema_body(m.ss[w.i], w.blk, run);
 }
 
 // ------------------------------------------------------------ grid rebuild
@@ -4595,7 +4638,7 @@ void enqueue_schema(const Seq &q)
             k_collect<<<grid_for(q.one->s.node_cap), kBlock, 0, q.one->stream>>>(q.one->s);
         });
     step(
-        q, K_SCHEMA, [](const glint_ctx &) -> uint32_t { return 1; },
+        q, K_SCHEMA, [&](const glint_ctx &) -> uint32_t { return q.one ? kSchemaBlocks : kSchemaBlocksFused; },
         [&](hipStream_t st, uint32_t g, glint_ctx &c) { k_schema<<<g, kSchemaThreads, 0, st>>>(c.s, q.run); },
         [&](hipStream_t st, uint32_t g, const Many &m) { kf_schema<<<g, kSchemaThreads, 0, st>>>(m, q.run); });
 }
