@@ -3781,6 +3781,7 @@ struct TableLds {
     float4 sbox[KV ? NT / 64 : 1][KV ? kMeetStage : 1];   // the staged meetings' boxes
     uint32_t staged[NT / 64], logged[NT / 64];            // every wave's staged meetings, and those in the map box
     unsigned long long meet_at, log_at;                   // the workgroup's places for them
+    unsigned long long ring;                              // where the tick's first goes in the meeting log
     uint32_t dups;
 };
 
@@ -3801,18 +3802,30 @@ __device__ __forceinline__ uint32_t meetings_in_map(const DevState &s, const flo
     return total;
 }
 
+// at % cap by subtraction (a tick's meetings mostly wrap a ring once; the
+// compiler's division held a dozen registers wherever meetings are written).
+__device__ __forceinline__ unsigned long long ring_place(unsigned long long at, unsigned long long cap)
+{
+    while (at >= cap) {
+        unsigned long long c = cap;
+        while (c <= at >> 1) c <<= 1;
+        at -= c;
+    }
+    return at;
+}
+
 // A wave's staged meetings written at place b of the tick's meetings (and of
 // the meeting log ring, whose total the end of the tick advances), those in
 // the map box also at place k of the key-value log.
 template <bool KV>
 __device__ __forceinline__ void table_store(const DevState &s, const glint_meeting *st, const float4 *sb, uint32_t nst,
-                                            unsigned long long b, unsigned long long k)
+                                            unsigned long long b, unsigned long long k, unsigned long long ring)
 {
     const uint32_t lane = lane_id();
     for (uint32_t j = lane; j < nst; j += 64) {
         if (b + j < s.meet_cap) {
             s.meet[b + j] = st[j];
-            if (s.mlog) s.mlog[(s.ctr->n_mlog + b + j) % s.mlog_cap] = st[j];
+            if (s.mlog) s.mlog[ring_place(ring + b + j, s.mlog_cap)] = st[j];
         } else {
             atomicOr(&s.ctr->error, kErrMeetCap);
         }
@@ -3844,7 +3857,7 @@ __device__ __forceinline__ void table_store(const DevState &s, const glint_meeti
 // A wave whose stage is full writes its meetings out alone.
 template <bool KV, int NT>
 __device__ __forceinline__ void table_flush_stage(const DevState &s, glint_meeting *st, const float4 *sb,
-                                                  uint32_t &nst)
+                                                  uint32_t &nst, unsigned long long ring)
 {
     wave_sync();
     const uint32_t lane = lane_id();
@@ -3855,7 +3868,7 @@ __device__ __forceinline__ void table_flush_stage(const DevState &s, glint_meeti
         if (lane == 0 && logged) k = atomicAdd(&s.ctr->n_kvlog, (unsigned long long)logged);
         k = __shfl(k, 0);
     }
-    table_store<KV>(s, st, sb, nst, __shfl(b, 0), k);
+    table_store<KV>(s, st, sb, nst, __shfl(b, 0), k, ring);
     wave_sync();
     nst = 0;
 }
@@ -3891,7 +3904,7 @@ __device__ __forceinline__ void table_flush_group(const DevState &s, TableLds<KV
         if (threadIdx.x == 0 && lall) L.log_at = atomicAdd(&s.ctr->n_kvlog, (unsigned long long)lall);
         lds_barrier();
     }
-    table_store<KV>(s, st, sb, nst, L.meet_at + before, L.log_at + lbefore);
+    table_store<KV>(s, st, sb, nst, L.meet_at + before, L.log_at + lbefore, L.ring);
     nst = 0;
 }
 
@@ -3965,7 +3978,7 @@ __device__ __forceinline__ void table_old(TableLds<KV, NT> &L, const DevState &s
         if constexpr (KV) sb[at] = s.tp->mbr_old[i];   // the run's box, logged when the stage is written
     }
     nst += (uint32_t)__popcll(m);
-    if (nst > kMeetStage - 64) table_flush_stage<KV, NT>(s, st, sb, nst);
+    if (nst > kMeetStage - 64) table_flush_stage<KV, NT>(s, st, sb, nst, L.ring);
 }
 
 // Start (and, with the key-value output, box) of contact c, whose hash slot
@@ -4077,7 +4090,10 @@ __device__ __forceinline__ void table_body(const DevState s, const P blk)
         }
     };
     if (blk.id() >= nreg) return;
-    if (threadIdx.x == 0) L.dups = 0;   // (the regions' barriers come before its use)
+    if (threadIdx.x == 0) {   // (the regions' barriers come before their use)
+        L.dups = 0;
+        if (s.mlog) L.ring = s.ctr->n_mlog % s.mlog_cap;
+    }
     bounds(blk.id());
     prefetch(blk.id());
     for (uint32_t r = blk.id(); r < nreg; r += blk.count()) {
