@@ -4654,7 +4654,11 @@ void enqueue_schema(const Seq &q)
             k_collect<<<grid_for(q.one->s.node_cap), kBlock, 0, q.one->stream>>>(q.one->s);
         });
     step(
-        q, K_SCHEMA, [&](const glint_ctx &) -> uint32_t { return q.one ? kSchemaBlocks : kSchemaBlocksFused; },
+        q, K_SCHEMA,
+        [&](const glint_ctx &c) -> uint32_t {
+            if (c.cfg.dynamic_schema != GLINT_SCHEMA_DYNAMIC) return 1;   // (the totals and the stamp alone)
+            return q.one ? kSchemaBlocks : kSchemaBlocksFused;
+        },
         [&](hipStream_t st, uint32_t g, glint_ctx &c) { k_schema<<<g, kSchemaThreads, 0, st>>>(c.s, q.run); },
         [&](hipStream_t st, uint32_t g, const Many &m) { kf_schema<<<g, kSchemaThreads, 0, st>>>(m, q.run); });
 }
