@@ -72,7 +72,9 @@ constexpr uint32_t kQueueSchema = 32, kQueueWords = 48;
 constexpr uint64_t kOrderMeetings = 2048;
 constexpr uint32_t kMaxJoinBlocks = 1024;           // workgroups of a context's join at most
 constexpr uint32_t kHeavyLeaf = 256;                // leaves above this size are joined first
-constexpr uint32_t kSparseMax = 512;                // most objects of a leaf joined by one wave
+// Most objects of a leaf joined by one wave: what its LDS holds (with 256, 7M
+// uniform objects in leaves of up to 512 take 11.1 ms where they take 5.4).
+constexpr uint32_t kSparseMax = 512;
 // and most objects per reach x reach square of it.  Denser leaves have
 // several contacts per object, which a wave decides one gather at a time and
 // the tiles in LDS: at 10M objects in hotspots a pass of 8 ticks takes 58.6 ms
@@ -1901,8 +1903,9 @@ __device__ __forceinline__ void lookup_body(const DevState s, const P blk)
 // lookup waits on chains of node reads and the scatter moves bytes.  A third
 // of the workgroups look up, first in the launch since theirs are the longer
 // waits (alternating them with the scatter's takes 3% longer at 10M objects
-// and in 32 cities).  Together 56 us at 1M uniform objects (48 + 19 apart),
-// 0.85 ms at 10M in hotspots (0.52 + 0.36).
+// and in 32 cities).  Together 56 us at 1M uniform objects when every lane still
+// walked alone (48 + 19 apart), 32 with the shared walk; 0.81 ms at 10M in
+// hotspots (0.52 + 0.36 apart).
 constexpr uint32_t kPlaceMax = 8192;
 __host__ __device__ inline uint32_t scatter_blocks(uint32_t n)
 {
@@ -1955,17 +1958,18 @@ __global__ __launch_bounds__(kBlock) void kf_unit_scatter(const Many m)
 
 // ------------------------------------------------------------ meeting table
 //
-// The table is an open-addressed hash of the pair key (pid_lo << 32) | pid_hi
-// in two generations of B 16-byte slots.  h = pair_hash(key): the high bits pick
-// a region of kRegion slots, the 11 bits below them the home slot inside it,
-// and linear probing wraps inside the region.  A tick's contacts are bucketed by region
-// and every region is then updated by one workgroup in LDS: the region of the
-// previous generation is read once, the new region is written once.
+// The meetings in progress are the contact list of the last tick, grouped by
+// region, with a start tick beside every entry (k_table; two generations, taken
+// in turn).  pair_hash of the pair key (pid_lo << 32) | pid_hi gives an entry its
+// region by its high bits and its home slot in the region's LDS hash by the 11
+// bits below them; linear probing wraps inside the region.  A tick's contacts
+// are bucketed by region and every region is then updated by one workgroup in
+// LDS: the region of the previous generation is read once, the new region is
+// written once.
 
-// The join writes the tick's contacts where the first bucketing pass reads
-// them: into the current generation's list when there are two passes (the
-// second pass writes the grouped list back there), else into the bucketing
-// buffer (the one pass writes the grouped list into the generation).
+// The join writes the tick's contacts into the current generation's list.  Two
+// bucketing passes go from there to clist2 and back; a list of one tile is
+// grouped in place (one_tile).
 __device__ __forceinline__ unsigned long long *contact_out(const DevState &s)
 {
     return s.tp->tab_cur.keys;
@@ -2005,10 +2009,10 @@ struct TableShape {
 // fewer regions and more only when pass 2 could not split the rest.  Pass 1
 // then writes runs of 64 contacts of a tile, pass 2 of 12288 over the regions
 // of a bin.  128 / 256 / 512 / 1024 bins (us of 8 ticks): 10M objects in
-// hotspots, 2^17 regions, 53200 / 51200 / 51200 / 51600 (pass 1 takes 400, 460
-// and 535 us a tick, pass 2 655, 590 and 575); 2M with the grid rebuild 10900 /
-// 10740 / 10790 / 10960; 400k in hotspots with key-value flush 4720 / 4750 /
-// 4820 / 4960.
+// hotspots, 2^17 regions, 53200 / 51200 / 51200 / 51600, where runs differ by
+// some 500 (pass 1 takes 400, 460 and 535 us a tick with 256, 512 and 1024, pass 2
+// 655, 590 and 575); 2M with the grid rebuild 10900 / 10740 / 10790 / 10960; 400k
+// in hotspots with key-value flush 4720 / 4750 / 4820 / 4960.
 __host__ __device__ inline uint32_t coarse_bits(uint32_t bits)
 {
     static_assert(kMaxFine == 2048 && kMaxRegionBits - 11 <= 10, "2^11 fine bins, at most 2^10 coarse ones");
@@ -2695,12 +2699,12 @@ struct JoinLds {
 // of it has to be taken back: those that the stage has no room for wait in
 // memory (SparseWave::past).  Ticks in us where the tiles join every leaf / no
 // leaf is handed over / as it is: 320 objects in one spot of a kilometre 320 /
-// 1230 / 311, 160 there 160 / 356 / 130, 40 there 106 / 75 / 76, 400 over 100 m of
-// two kilometres 132 / 267 / 102, 500 objects beside 12 of another leaf 590 / 3290
-// / 540, 120 in one spot among 100k uniform ones 305 / 258 / 142, 100k in spots of
-// 100 447 / 801 / 351, of 20 331 / 258 / 245 (at 1000 pairs 228, at 2000 267), of 5
-// 348 / 161 / 161, 1M in hotspots 1036 / 595 / 600; 256 leaves of 300 over 100 m
-// 194 / 157 / 119 (at 448 columns 180).
+// 1215 / 286, 160 there 160 / 368 / 131, 40 there 106 / 78 / 76, 400 over 100 m of
+// two kilometres 132 / 267 / 103, 500 objects beside 12 of another leaf 585 / 3290
+// / 580, 120 in one spot among 100k uniform ones 305 / 257 / 140, 100k in spots of
+// 100 445 / 797 / 348, of 20 333 / 257 / 245 (at 1000 pairs 228, at 2000 267), of 5
+// 344 / 160 / 161, 1M in hotspots 1040 / 597 / 598; 256 leaves of 300 over 100 m
+// 192 / 155 / 120 (at 448 columns 180).
 // A leaf of 100 objects takes a wave about 5 us, nearly all of it waiting:
 // the leaf's record and positions (2 us), the sort (1.3), the runs (1.7).
 // The join of 1M uniform objects went from 297 to 39 us, of 300k in lon/lat
@@ -2729,7 +2733,7 @@ struct JoinSums {
 };
 
 struct SparseLds {
-    float2 pos[kSparseMax + 1];           // offsets from the leaf's low corner in reaches, cell order, and one beyond reach
+    float2 pos[kSparseMax + 1];           // offsets from the low corner in reaches, cell order, and one beyond reach
     float2 pad;                           // (start is read 16 bytes at a time)
     uint16_t at[kSparseMax];              // their place in the leaf's run of the sorted arrays
     uint32_t start[kSparseCells + 4];     // first object of every cell, and the count at the end
@@ -2846,8 +2850,8 @@ __device__ __forceinline__ void sparse_drain(const DevState &s, const TickView &
 // False for a leaf that is left to the tiles: none of its pairs is staged then.
 // few: at most kSparseFew leaves are sparse.
 template <bool GEO>
-__device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &tv, SparseLds &L,
-                                            SparseWave &w, uint32_t leaf, bool few)
+__device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &tv, SparseLds &L, SparseWave &w,
+                                            uint32_t leaf, bool few)
 {
     const uint32_t lane = lane_id(), before_leaf = w.n;
     const uint32_t off = s.offset[leaf], cnt = s.count[leaf];
@@ -2952,8 +2956,8 @@ __device__ __forceinline__ bool join_sparse(const DevState &s, const TickView &t
             for (uint32_t q = 0; q < kSparseCols; q++) {
                 if (!m[q]) continue;
                 if (__builtin_amdgcn_inverse_ballot_w64(m[q])) {
-                    const uint32_t place = w.n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m[q] >> 32),
-                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m[q], 0u));
+                    const uint32_t below_lane = __builtin_amdgcn_mbcnt_lo((uint32_t)m[q], 0u);
+                    const uint32_t place = w.n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m[q] >> 32), below_lane);
                     const uint2 e = make_uint2(ex, (off + L.at[j[q]]) | flag);
                     if (place < kSparseStage)
                         L.stage[place] = e;

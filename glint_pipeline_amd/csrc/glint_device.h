@@ -255,7 +255,7 @@ struct DevState {
     float *pfx;             // positions at the tick before as FP32 offsets from the same corner
     float *pfy;             // (NaN beyond pf_lim: left to the FP64 test)
     glint_meeting *meet;
-    unsigned long long *clist2;    // bucketing buffer (the join's output when there is one pass)
+    unsigned long long *clist2;    // what pass 1 of the bucketing writes (before it, a share per wave of the join)
     uint32_t *bins;                // contacts per coarse bin, a line each
     uint32_t *boff;                // per coarse bin and bucketing block: its place in the bin
     uint32_t rbits_min;            // log2(regions) of the configured table: the fewest a tick uses

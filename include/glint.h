@@ -131,7 +131,10 @@ typedef struct glint_tick_stats {
     uint64_t num_meetings;         /* meetings emitted this tick */
     uint64_t num_rechecks;         /* FP64 rechecks (FP32 guard mode) */
     uint64_t table_slots;
-    float ms_partition, ms_lookup, ms_refine, ms_evaluate, ms_schema;  /* HIP event times */
+    /* HIP event times of the stage calls' last tick: the assignment and the leaves' offsets; the
+     * counting sort by leaf with the lookup, and the units grouped by leaf; the join and the
+     * grouping of its contacts; the meeting table; the schema update */
+    float ms_partition, ms_lookup, ms_refine, ms_evaluate, ms_schema;
     uint64_t num_stored;           /* contacts kept in the meeting table's generation */
     uint64_t ref_drop_objects;     /* objects beyond 2*grid_capacity in their leaf: the reference
                                       stores at most that many per leaf and drops the rest in
