@@ -2,8 +2,8 @@
  * oracle.h - CPU restatement of GLINT's per-tick contact-tracing path.
  *
  * TEST INFRASTRUCTURE ONLY.  Only tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py may load this library, and only as the checker
- * or as the reported CPU baseline.  The product (libglint.so) never links,
+ * cpu_baseline leg of bench.py may load this library, and only to compare
+ * with it or as the reported CPU baseline.  The product (libglint.so) never links,
  * loads or calls it.
  *
  * What it restates (reference paths relative to the reference repository):
